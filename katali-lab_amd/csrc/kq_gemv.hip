@@ -2,13 +2,23 @@
 // activations), per-block integer sums, synthetic data and a copy kernel.
 //
 // GEMV layout: a row is nb = cols/256 super-blocks = nb*IPB lane items. S lanes
-// (a power of two dividing the item count, at most 64) share a row and each
-// takes IPL = items/S items (item = s + S*i, so a wave instruction walks
-// consecutive items of a row). A wave holds 64/S rows at a time, a 256-thread
-// workgroup 4x that, and each slot issues the loads of RPS rows before it
-// computes any of them. The activation is staged once per workgroup in LDS.
+// (a power of two, at most 64) share a row and each takes N items of it per
+// batch (item = s + S*i, so a wave instruction walks consecutive items of a
+// row; gemv_shape picks S and N). A wave holds 64/S rows at a time and each
+// slot issues the loads of RPS rows, N items each, before it computes any of
+// them. The activation is staged once per workgroup in LDS, in item order.
+//
+// Bound by the weight stream for large matrices (Q6_K 151936 x 2048, q8_1:
+// 48.2 us, 5.3 TB/s, before the quad loads 50.6; Q4_K with an fp32 activation
+// by its converts and FMAs, about 110 per 18 bytes: 40000 x 5120 4.0 TB/s), by
+// launch, first loads and tail below about 20 MB. Row lengths that are no
+// power of two used to run a loop over items with one load in flight and as
+// few as 4 lanes per row (Q6_K 5120 x 13824, fp32: 50.4 us, now 19.9; Q4_K
+// 9731 x 2560: 8.9, now 5.6; q, k, v of 2560 columns: 10.1, now 6.5).
 #include "kq_device.h"
 #include "kq_launch.h"
+
+#include <type_traits>
 
 namespace kq {
 
@@ -49,23 +59,144 @@ hipError_t launch_quantize_q8_1(const float *x, uint64_t n, uint8_t *out, hipStr
 // ---------------------------------------------------------------------------
 // GEMV
 // ---------------------------------------------------------------------------
-// The activation of a GEMV workgroup, staged in two halves around the weight
-// loads: load() issues the first XPRE tasks per thread into registers (the
-// whole activation for cols <= 4096), store() writes them to LDS after the
-// weight loads are out and stages any remaining tasks directly. A task is 4
-// values: fp32 copied (MODE 0), q8_1 bytes copied (MODE 1), or fp32
-// quantized to q8_1 with 8 lanes per block (MODE 2).
+// The activation of a GEMV workgroup in LDS, laid out for the lanes that read
+// it. A lane item takes NQ groups of 16 values (Q4_K: sub-blocks 2g and 2g+1;
+// Q6_K: quarters t = 0..3 of a half). Tiles of 16 items hold word after word
+// of each group side by side for the 16 items, so the lanes of a row read
+// consecutive 16-byte words at offsets the instruction carries; in the
+// activation's own order they are 64 (fp32) or up to 128 (q8_1) bytes apart,
+// a 4-way bank conflict on every read.
+//   MODE 0     float4 [4 NQ words][16 items], then the groups' sums (left to
+//              right) float [NQ][16]; words 288 bytes apart, so that the eight
+//              lanes storing one 32-value run hit distinct banks
+//   MODE 1, 2  int8 x 16 [NQ][16], the q8_1 blocks' d float [NQ][8], the
+//              groups' exact sums int [NQ][16]
+template <class QT, int MODE>
+struct XLds {
+    static constexpr uint32_t NQ = 16 / QT::IPB;
+    static constexpr uint32_t WORD = MODE == 0 ? 288 : 256;
+    static constexpr uint32_t D8 = NQ * WORD, SUM = MODE == 0 ? 4 * NQ * WORD : D8 + NQ * 32;
+    static constexpr uint32_t TILE = (SUM + NQ * 64 + 127) & ~127u;   // whole rows of banks
+    static constexpr uint32_t bytes(uint32_t items) { return (items + 15) / 16 * TILE; }
+    // the item and group of 16-value run h (counted along the activation)
+    __device__ static __forceinline__ void place(uint32_t h, uint32_t &item, uint32_t &q) {
+        if constexpr (QT::TYPE == T_Q4_K) {   // h = 16 b + 4 g + 2 q + hh
+            q = (h >> 1) & 1;
+            item = ((h >> 2) << 1) | (h & 1);
+        } else {                              // h = 16 b + 8 n + 2 q + k
+            q = (h >> 1) & 3;
+            item = ((h >> 3) << 1) | (h & 1);
+        }
+    }
+    uint8_t *t;   // the item's tile
+    uint32_t l;   // the item in it
+    __device__ __forceinline__ XLds(uint8_t *lds, uint32_t item) : t(lds + (item >> 4) * TILE), l(item & 15) {}
+    __device__ __forceinline__ float4 *xf(uint32_t word) const { return (float4 *)(t + word * WORD + l * 16); }
+    __device__ __forceinline__ float *fsum(uint32_t q) const { return (float *)(t + SUM + q * 64 + l * 4); }
+    __device__ __forceinline__ int4 *xq(uint32_t q) const { return (int4 *)(t + q * WORD + l * 16); }
+    __device__ __forceinline__ float *d8(uint32_t q) const { return (float *)(t + D8 + q * 32 + (l >> 1) * 4); }
+    __device__ __forceinline__ int *isum(uint32_t q) const { return (int *)(t + SUM + q * 64 + l * 4); }
+};
+
+// Rows a lane slot loads together, by the items each lane takes of a row, and
+// the most items per batch (Q4_K: 8 VGPRs of raw block each, Q6_K: 14).
+template <class QT>
+constexpr int gemv_rps(int n) {
+    return QT::TYPE == T_Q4_K ? (n == 1 ? 4 : (n == 2 ? 2 : 1)) : (n == 1 ? 2 : 1);
+}
+template <class QT>
+constexpr int gemv_nmax() { return QT::TYPE == T_Q4_K ? 8 : 5; }
+constexpr int GEMV_MAX_NT = 512;
+constexpr uint32_t GEMV_MAX_COLS = 32768;
+
+// fp32 contribution of one lane item (chunk c of a block) against the staged
+// activation: the block formats' own arithmetic (Q4K, Q6K in kq_device.h),
+// the activation read through XLds.
+template <int MODE>
+__device__ __forceinline__ float item_dot(const Q4K::Raw &r, int c, const XLds<Q4K, MODE> &x) {
+    const int g = c >> 1;
+    float ds0, ds1, dm0, dm1;
+    Q4K::scales(r, g, ds0, ds1, dm0, dm1);
+    if constexpr (MODE == 0) {
+        const uint32_t q[4] = {r.q.x, r.q.y, r.q.z, r.q.w};
+        float al = 0.0f, ah = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float4 vl = *x.xf(j), vh = *x.xf(4 + j);
+            const uint32_t lo = q[j] & 0x0F0F0F0Fu, hi = (q[j] >> 4) & 0x0F0F0F0Fu;
+            al = fmaf((float)(lo & 0xFFu), vl.x, al);
+            al = fmaf((float)((lo >> 8) & 0xFFu), vl.y, al);
+            al = fmaf((float)((lo >> 16) & 0xFFu), vl.z, al);
+            al = fmaf((float)(lo >> 24), vl.w, al);
+            ah = fmaf((float)(hi & 0xFFu), vh.x, ah);
+            ah = fmaf((float)((hi >> 8) & 0xFFu), vh.y, ah);
+            ah = fmaf((float)((hi >> 16) & 0xFFu), vh.z, ah);
+            ah = fmaf((float)(hi >> 24), vh.w, ah);
+        }
+        return fmaf(ds0, al, -(dm0 * *x.fsum(0))) + fmaf(ds1, ah, -(dm1 * *x.fsum(1)));
+    } else {
+        int slo, shi;
+        Q4K::isums_x(r.q, *x.xq(0), *x.xq(1), slo, shi);
+        const float vlo = fmaf(ds0, (float)slo, -(dm0 * (float)*x.isum(0)));
+        const float vhi = fmaf(ds1, (float)shi, -(dm1 * (float)*x.isum(1)));
+        return fmaf(*x.d8(0), vlo, *x.d8(1) * vhi);
+    }
+}
+template <int MODE>
+__device__ __forceinline__ float item_dot(const Q6K::Raw &r, int c, const XLds<Q6K, MODE> &x) {
+    const int k = c & 1;
+    const uint32_t A[4] = {r.A.x, r.A.y, r.A.z, r.A.w};
+    const uint32_t B[4] = {r.B.x, r.B.y, r.B.z, r.B.w};
+    const uint32_t H[4] = {r.H.x, r.H.y, r.H.z, r.H.w};
+    const float d = h2f(r.d);
+    float acc = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        if constexpr (MODE == 0) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t v = Q6K::q6(A[j], B[j], H[j], t);
+                const float4 w = *x.xf(4 * t + j);
+                s = fmaf((float)(v & 0xFFu), w.x, s);
+                s = fmaf((float)((v >> 8) & 0xFFu), w.y, s);
+                s = fmaf((float)((v >> 16) & 0xFFu), w.z, s);
+                s = fmaf((float)(v >> 24), w.w, s);
+            }
+            s = fmaf(-32.0f, *x.fsum(t), s);
+            acc = fmaf(d * Q6K::scale(r, k, t), s, acc);
+        } else {
+            const int4 w = *x.xq(t);
+            int s = dot4(Q6K::q6(A[0], B[0], H[0], t), w.x, 0);
+            s = dot4(Q6K::q6(A[1], B[1], H[1], t), w.y, s);
+            s = dot4(Q6K::q6(A[2], B[2], H[2], t), w.z, s);
+            s = dot4(Q6K::q6(A[3], B[3], H[3], t), w.w, s);
+            s -= 32 * *x.isum(t);
+            const float v = (d * Q6K::scale(r, k, t)) * (float)s;
+            acc = t == 0 ? *x.d8(t) * v : fmaf(*x.d8(t), v, acc);
+        }
+    }
+    return acc;
+}
+
+// The activation, staged in two halves around the weight loads: load() issues
+// the first XPRE tasks per thread into registers (the whole activation for
+// cols <= 4096 in 256 threads), store() writes them to LDS after the weight
+// loads are out and stages any remaining tasks directly. A task is 4 values:
+// fp32 copied (MODE 0), q8_1 bytes copied (MODE 1), or fp32 quantized to q8_1
+// with 8 lanes per block (MODE 2).
 constexpr int XPRE = 4;
-template <int MODE, uint32_t NT = 256>
+template <class QT, int MODE>
 struct XStage {
+    using X = XLds<QT, MODE>;
     float4 v[XPRE];
     uint32_t q[XPRE], d[XPRE];
-    __device__ static uint32_t tasks(uint32_t cols) { return MODE == 0 ? cols / 4 : cols / 32 * 8; }
     __device__ __forceinline__ void load(const float *xf, const uint8_t *xq, uint32_t cols) {
-        const uint32_t n = tasks(cols);
+        const uint32_t n = cols / 4, nt = blockDim.x;
 #pragma unroll
         for (int i = 0; i < XPRE; i++) {
-            const uint32_t t = min(threadIdx.x + NT * i, n - 1);   // clamped, not skipped
+            if (nt * i >= n) break;                                // uniform
+            const uint32_t t = min(threadIdx.x + nt * i, n - 1);   // clamped, not skipped
             if constexpr (MODE == 1) {
                 const uint8_t *b = xq + (t >> 3) * 36;
                 q[i] = *(const uint32_t *)(b + 4 + 4 * (t & 7));
@@ -77,12 +208,13 @@ struct XStage {
             }
         }
     }
-    __device__ __forceinline__ void put(uint32_t t, float4 x4, uint32_t qq, uint32_t dd, const Act &a,
-                                        const ActF &af) const {
+    __device__ __forceinline__ void put(uint32_t t, float4 x4, uint32_t qq, uint32_t dd, uint8_t *lds) const {
+        uint32_t item, grp;
+        X::place(t >> 2, item, grp);
+        const X x(lds, item);
         if constexpr (MODE == 0) {
-            *(float4 *)(af.x + 4 * t) = x4;
+            *x.xf(4 * grp + (t & 3)) = x4;
         } else {
-            const uint32_t blk = t >> 3, part = t & 7;
             uint32_t qv;
             int lo, hi;
             float dec;
@@ -94,26 +226,24 @@ struct XStage {
                 uint32_t d16, s16;
                 qv = quant_q8_1_part(x4, d16, s16, lo, hi, dec);
             }
-            *(uint32_t *)(a.qs + 32 * blk + 4 * part) = qv;
-            if (part == 0) {
-                a.d8[blk] = dec;
-                a.qs16[2 * blk] = lo;
-                a.qs16[2 * blk + 1] = hi;
+            ((uint32_t *)x.xq(grp))[t & 3] = qv;
+            if ((t & 3) == 0) {   // parts 0 and 4 of the block: its two halves, one item each
+                *x.isum(grp) = (t & 4) ? hi : lo;
+                *x.d8(grp) = dec;
             }
         }
     }
     // Tasks past n were loaded clamped and are dropped here (whole 8-lane
     // groups: n % 8 == 0); the barriers around the weight loads keep the
     // compiler from sinking the preloads into these branches.
-    __device__ __forceinline__ void store(const float *xf, const uint8_t *xq, uint32_t cols, const Act &a,
-                                          const ActF &af) const {
-        const uint32_t n = tasks(cols);
+    __device__ __forceinline__ void store(const float *xf, const uint8_t *xq, uint32_t cols, uint8_t *lds) const {
+        const uint32_t n = cols / 4, nt = blockDim.x;
 #pragma unroll
         for (int i = 0; i < XPRE; i++) {
-            const uint32_t t = threadIdx.x + NT * i;
-            if (t < n) put(t, v[i], q[i], d[i], a, af);
+            const uint32_t t = threadIdx.x + nt * i;
+            if (t < n) put(t, v[i], q[i], d[i], lds);
         }
-        for (uint32_t t = threadIdx.x + NT * XPRE; t < n; t += NT) {   // whole 8-lane groups (n % 8 == 0)
+        for (uint32_t t = threadIdx.x + nt * XPRE; t < n; t += nt) {   // whole 8-lane groups (n % 8 == 0)
             float4 x4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             uint32_t qq = 0, dd = 0;
             if constexpr (MODE == 1) {
@@ -123,144 +253,145 @@ struct XStage {
             } else {
                 x4 = *(const float4 *)(xf + 4 * t);
             }
-            put(t, x4, qq, dd, a, af);
+            put(t, x4, qq, dd, lds);
         }
         if constexpr (MODE == 0) {   // half-block sums of the fp32 activation
             __syncthreads();
-            for (uint32_t t = threadIdx.x; t < cols / 16; t += NT) {
+            for (uint32_t h = threadIdx.x; h < cols / 16; h += nt) {
+                uint32_t item, grp;
+                X::place(h, item, grp);
+                const X x(lds, item);
                 float sum = 0.0f;
-                for (int i = 0; i < 16; i++) sum += af.x[16 * t + i];
-                af.xs16[t] = sum;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float4 w = *x.xf(4 * grp + j);
+                    sum += w.x;
+                    sum += w.y;
+                    sum += w.z;
+                    sum += w.w;
+                }
+                *x.fsum(grp) = sum;
             }
         }
     }
 };
 
 // The row groups of one matrix that workgroup `block` of `nblocks` takes
-// (the workgroups' shares of the matrix interleave: a grid-stride loop);
-// NW waves per workgroup.
-template <class QT, int IPL_T, int RPS, int MODE, int NW = 4>
+// (the workgroups' shares of the matrix interleave: a grid-stride loop). The
+// S lanes of a row take items s, s + S, ... in batches of N, all of a batch's
+// loads in flight at once; items past the row's end load the last one and
+// count as zero.
+template <class QT, int N, int RPS, int MODE>
 __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_t rows, uint32_t cols, uint64_t rb,
                                           uint32_t log2s, const float *xf, const uint8_t *xq, float *__restrict__ y,
                                           uint32_t block, uint32_t nblocks, uint8_t *lds) {
-    const Act a = act_carve(lds, cols);
-    const ActF af = actf_carve(lds, cols);
     const uint32_t S = 1u << log2s;
     const uint32_t slots = WAVE >> log2s;
-    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, NW = blockDim.x / WAVE;
     const uint32_t slot = lane >> log2s, s = lane & (S - 1);
     const uint32_t items = cols / 256 * QT::IPB;
-    const int IPL = IPL_T > 0 ? IPL_T : (int)(items >> log2s);
     const uint32_t rows_iter = NW * slots * RPS;
     const uint32_t base0 = block * rows_iter;
     auto row_of = [&](uint32_t base, int r) { return base + r * (NW * slots) + wave * slots + slot; };
 
-    // Unrolled items: the activation loads, then the first row group's
-    // weight loads, go out before the activation is staged, so the two
-    // latencies overlap. Rows are clamped,
-    // not skipped (a load under a branch makes the compiler wait for all).
-    typename QT::Raw raw[RPS][IPL_T > 0 ? IPL_T : 1];
-    auto load_rows = [&](uint32_t base) {
-        if constexpr (IPL_T > 0) {
+    // The activation loads, then the first row group's weight loads, go out
+    // before the activation is staged, so the two latencies overlap. Rows are
+    // clamped, not skipped (a load under a branch makes the compiler wait for
+    // all).
+    typename QT::RawQ raw[RPS][N];   // (a quad's lanes hold one block's items, or all lie past the row)
+    auto load_rows = [&](uint32_t base, uint32_t i0) {
 #pragma unroll
-            for (int r = 0; r < RPS; r++) {
-                const uint8_t *rp = w + (uint64_t)min(row_of(base, r), rows - 1) * rb;
+        for (int r = 0; r < RPS; r++) {
+            const uint8_t *rp = w + (uint64_t)min(row_of(base, r), rows - 1) * rb;
 #pragma unroll
-                for (int i = 0; i < IPL_T; i++) {
-                    const uint32_t item = s + S * i;
-                    raw[r][i] = QT::load(rp + (item / QT::IPB) * QT::BB, item % QT::IPB);
-                }
+            for (int i = 0; i < N; i++) {
+                const uint32_t item = min(s + S * (i0 + i), items - 1);
+                raw[r][i] = QT::load_quad(rp + (item / QT::IPB) * QT::BB, item % QT::IPB);
             }
         }
     };
-    XStage<MODE, 64 * NW> xs;
+    XStage<QT, MODE> xs;
     xs.load(xf, xq, cols);   // issued first: waiting for x then waits for nothing else
     // Neither the compiler nor the scheduler may move work across these two
     // points (x is deliberately not __restrict__, so its loads are not
     // treated as invariant and re-issued at their use).
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    load_rows(base0);   // base0 < rows: the grid never exceeds the row groups
+    load_rows(base0, 0);   // base0 < rows: the grid never exceeds the row groups
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);   // every weight load is out before x is staged
-    xs.store(xf, xq, cols, a, af);
+    xs.store(xf, xq, cols, lds);
     __syncthreads();
 
-    for (uint32_t base = base0; base < rows; base += nblocks * rows_iter) {
-        float acc[RPS];
-        if constexpr (IPL_T > 0) {
-            if (base != base0) load_rows(base);
+    float acc[RPS];
+#pragma unroll
+    for (int r = 0; r < RPS; r++) acc[r] = 0.0f;
+    for (uint32_t base = base0, i0 = 0;;) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const uint32_t at = s + S * (i0 + i), item = min(at, items - 1);
+            const XLds<QT, MODE> x(lds, item);
 #pragma unroll
             for (int r = 0; r < RPS; r++) {
-                float v = 0.0f;
-#pragma unroll
-                for (int i = 0; i < IPL_T; i++) {
-                    const uint32_t item = s + S * i;
-                    if constexpr (MODE == 0) v += QT::dot_f32(raw[r][i], item % QT::IPB, af, item / QT::IPB);
-                    else v += QT::dot_q8(raw[r][i], item % QT::IPB, a, item / QT::IPB);
-                }
-                acc[r] = v;
+                const float v = item_dot<MODE>(QT::full(raw[r][i]), item % QT::IPB, x);
+                acc[r] += at < items ? v : 0.0f;
             }
-        } else {
+            // The rows share an item's activation; the next item's is read
+            // when this one's dots are done (left alone, the compiler reads
+            // every item's first and keeps them in registers, or spills).
 #pragma unroll
-            for (int r = 0; r < RPS; r++) {
-                const uint32_t row = row_of(base, r);
-                float v = 0.0f;
-                if (row < rows) {
-                    const uint8_t *rp = w + (uint64_t)row * rb;
-                    for (int i = 0; i < IPL; i++) {
-                        const uint32_t item = s + S * i;
-                        const typename QT::Raw rw = QT::load(rp + (item / QT::IPB) * QT::BB, item % QT::IPB);
-                        if constexpr (MODE == 0) v += QT::dot_f32(rw, item % QT::IPB, af, item / QT::IPB);
-                        else v += QT::dot_q8(rw, item % QT::IPB, a, item / QT::IPB);
+            for (int r = 0; r < RPS; r++) asm volatile("" : "+v"(acc[r])::"memory");
+        }
+        i0 += N;
+        if (S * i0 >= items) {   // the row group is done
+            if (log2s == 6) {
+                // one row per wave instruction: the RPS rows reduce together
+                // (halving exchanges, no LDS); lane groups of 64 / RPS then
+                // hold row (lane >> SH) & (RPS - 1)
+                constexpr int LOGR = RPS >= 4 ? 2 : (RPS >= 2 ? 1 : 0);
+                constexpr int SH = 6 - LOGR;
+                const float v = reduce_rows<RPS>(acc);
+                const uint32_t r = (lane >> SH) & (RPS - 1);
+                const uint32_t row = row_of(base, (int)r);
+                if ((lane & ((1u << SH) - 1)) == 0 && row < rows) y[row] = v;
+            } else {
+#pragma unroll
+                for (int r = 0; r < RPS; r++) {
+                    float v;
+                    switch (log2s) {   // uniform: the lanes of a row slot sum on the VALU
+                        case 5: v = group_sum<32>(acc[r]); break;
+                        case 4: v = group_sum<16>(acc[r]); break;
+                        case 3: v = group_sum<8>(acc[r]); break;
+                        default: v = group_sum<4>(acc[r]); break;
                     }
+                    const uint32_t row = row_of(base, r);
+                    if (s == 0 && row < rows) y[row] = v;
                 }
-                acc[r] = v;
             }
-        }
-        if (log2s == 6) {
-            // one row per wave instruction: the RPS rows reduce together
-            // (halving exchanges, no LDS); lane groups of 64 / RPS then hold
-            // row (lane >> SH) & (RPS - 1)
-            constexpr int LOGR = RPS >= 4 ? 2 : (RPS >= 2 ? 1 : 0);
-            constexpr int SH = 6 - LOGR;
-            const float v = reduce_rows<RPS>(acc);
-            const uint32_t r = (lane >> SH) & (RPS - 1);
-            const uint32_t row = row_of(base, (int)r);
-            if ((lane & ((1u << SH) - 1)) == 0 && row < rows) y[row] = v;
-        } else {
+            base += nblocks * rows_iter;
+            if (base >= rows) break;
+            i0 = 0;
 #pragma unroll
-            for (int r = 0; r < RPS; r++) {
-                float v;
-                switch (log2s) {   // uniform: the lanes of a row slot sum on the VALU
-                    case 5: v = group_sum<32>(acc[r]); break;
-                    case 4: v = group_sum<16>(acc[r]); break;
-                    case 3: v = group_sum<8>(acc[r]); break;
-                    case 2: v = group_sum<4>(acc[r]); break;
-                    case 1: v = group_sum<2>(acc[r]); break;
-                    default: v = acc[r]; break;
-                }
-                const uint32_t row = row_of(base, r);
-                if (s == 0 && row < rows) y[row] = v;
-            }
+            for (int r = 0; r < RPS; r++) acc[r] = 0.0f;
         }
+        load_rows(base, i0);
     }
 }
 
-template <class QT, int IPL_T, int RPS, int MODE, int NW = 4>
-__global__ void __launch_bounds__(64 * NW)
+template <class QT, int N, int RPS, int MODE>
+__global__ void __launch_bounds__(GEMV_MAX_NT)
     k_gemv(const uint8_t *__restrict__ w, uint32_t rows, uint32_t cols, uint64_t rb, uint32_t log2s,
            const float *xf, const uint8_t *xq, float *__restrict__ y) {
     extern __shared__ __align__(16) uint8_t lds[];
-    gemv_rows<QT, IPL_T, RPS, MODE, NW>(w, rows, cols, rb, log2s, xf, xq, y, blockIdx.x, gridDim.x, lds);
+    gemv_rows<QT, N, RPS, MODE>(w, rows, cols, rb, log2s, xf, xq, y, blockIdx.x, gridDim.x, lds);
 }
 
 // Up to four GEMVs over one activation in one launch (the engine's
 // matvec_multi: q, k and v of a layer). Matrix m owns workgroups
 // [end[m-1], end[m]) and runs the single-matrix body on them, so each row's
 // arithmetic, and its bits, are those of k_gemv.
-template <int IPL4, int RPS4, int IPL6, int RPS6, int MODE>
-__global__ void __launch_bounds__(256) k_gemv_multi(GemvMultiArgs g) {
+template <int N4, int N6, int MODE>
+__global__ void __launch_bounds__(GEMV_MAX_NT) k_gemv_multi(GemvMultiArgs g) {
     extern __shared__ __align__(16) uint8_t lds[];
     uint32_t m = 0;
 #pragma unroll
@@ -269,11 +400,11 @@ __global__ void __launch_bounds__(256) k_gemv_multi(GemvMultiArgs g) {
     const uint32_t start = m ? g.end[m - 1] : 0;
     const uint32_t blk = blockIdx.x - start, nblk = g.end[m] - start;
     if (g.type[m] == T_Q4_K)
-        gemv_rows<Q4K, IPL4, RPS4, MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q4K::BB, g.log2s4,
-                                         g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q4K, N4, gemv_rps<Q4K>(N4), MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q4K::BB,
+                                                    g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
     else
-        gemv_rows<Q6K, IPL6, RPS6, MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q6K::BB, g.log2s6,
-                                         g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q6K, N6, gemv_rps<Q6K>(N6), MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q6K::BB,
+                                                    g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
 }
 
 static int ilog2(uint32_t v) {
@@ -282,101 +413,134 @@ static int ilog2(uint32_t v) {
     return l;
 }
 
-// S = largest power of two <= 64 dividing the item count.
-static uint32_t lanes_per_row(uint32_t items) {
-    uint32_t s = 64;
-    while (s > 1 && items % s) s >>= 1;
-    return s;
+// How a row's items are spread: S lanes (a power of two) take N items each
+// per batch. The widest S that takes the row in one batch (any batches for 64
+// lanes: rows past every S) and pads it by at most a quarter (items past the
+// row's end, computed and dropped), else by at most a third, else a half:
+// wide rows read longer runs per instruction, and leave a lane fewer items in
+// a chain and a small matrix more waves (Q4_K 9731 x 2560, 32 lanes x 3
+// items: 5.6 us, 16 x 5: 6.4; 5120 x 5120 6.5 and 7.7). A large matrix fills
+// the chip either way and pays for the padding instead, so there at most an
+// eighth comes first (Q4_K 20000 x 5120, 64 x 3: 14.5 us, 32 x 5: 13.0; Q6_K
+// 40000 x 5120 37.4 and 34.2).
+struct GemvShape {
+    uint32_t S, N;
+};
+constexpr GemvShape gemv_shape(uint32_t items, uint32_t nmax, bool large) {
+    for (uint32_t den = large ? 8 : 4; den >= 2; den = den == 8 ? 4 : den - 1)
+        for (uint32_t S = 64; S >= 4; S >>= 1) {
+            const uint32_t steps = (items + S - 1) / S, batches = (steps + nmax - 1) / nmax;
+            const uint32_t N = (steps + batches - 1) / batches;
+            if ((batches == 1 || S == 64) && den * S * N * batches <= (den + 1) * items) return {S, N};
+        }
+    return {64, nmax};
+}
+// large: from 6144 items per CU (between 0.8 and 2.4 million measured)
+template <class QT>
+constexpr GemvShape gemv_shape(uint64_t rows, uint64_t cols, uint64_t cus) {
+    const uint32_t items = (uint32_t)(cols / 256) * QT::IPB;
+    return gemv_shape(items, gemv_nmax<QT>(), rows > 6144 * cus / items);
+}
+// the item counts that the two formats have at one and the same row length
+constexpr bool gemv_pair(uint32_t n4, uint32_t n6) {
+    for (uint64_t cols = 256; cols <= GEMV_MAX_COLS; cols += 256)
+        if (gemv_shape<Q4K>(0, cols, 1).N == n4 && gemv_shape<Q6K>(0, cols, 1).N == n6) return true;
+    return false;
 }
 
-// Waves per workgroup of a single GEMV: the count (4, 6 or 8) whose grid
-// puts the fewest rows on the busiest CU (each CU streams at most ~25 GB/s,
-// so the busiest one sets the time), the smallest among equals. 6144 rows of
-// 16 per 4-wave workgroup are 384 workgroups, two on half of 256 CUs; 6
-// waves make 256 workgroups of 24 rows, one per CU.
-static int gemv_waves(uint64_t rows, uint32_t rows_per_wave, int cus) {
-    int best = 4;
-    uint64_t best_rows = ~0ull;
-    for (int nw : {4, 6, 8}) {
-        const uint64_t per = (uint64_t)nw * rows_per_wave;
-        const uint64_t iters = (rows + per - 1) / per;
-        const uint64_t busiest = (iters + cus - 1) / cus * per;
-        if (busiest < best_rows) best = nw, best_rows = busiest;
+// f(integral_constant<int, N>) for the run-time N in 1..MAX
+template <int MAX, class F>
+static hipError_t with_n(uint32_t n, F &&f) {
+    if constexpr (MAX > 1)
+        if (n < (uint32_t)MAX) return with_n<MAX - 1>(n, f);
+    return f(std::integral_constant<int, MAX>{});
+}
+
+// Waves per workgroup and the most workgroups per CU, for `waves` waves of
+// rows. Up to 16 waves per CU: the count (4, 6 or 8) that puts the fewest
+// waves on the busiest CU, which sets the time, the largest among equals
+// (fewer workgroups stage the activation): 6144 rows of 2048 columns in 6
+// waves make 256 workgroups, one per CU; 4096 x 4096 Q4_K takes 4.3 us in 256
+// workgroups of 8 waves, 4.9 in 512 of 4. Past that the workgroups loop over
+// their rows: above 2048 columns two resident ones of 8 waves, so that the
+// activation is staged twice per CU rather than once per 4 waves (Q6_K 5120 x
+// 13824: 20.3 against 26.0 us; Q4_K 9731 x 2560: 6.0 against 6.8), up to there
+// as many of 4 waves as fit (Q4_K 25000 x 1536: 6.5 against 7.1 us in 8
+// waves). Past 64 waves per CU each loops many times and four of 8 waves
+// keep more loads in flight (Q4_K 40000 x 4096: 22.9 against 23.5 us in two).
+struct GemvGrid {
+    uint32_t nw, cap;
+};
+static GemvGrid gemv_grid(uint64_t waves, uint64_t cols, uint32_t cus) {
+    if (waves > 64ull * cus) return {8, 4};
+    if (waves > 16ull * cus) return cols > 2048 ? GemvGrid{8, 2} : GemvGrid{4, 8};
+    GemvGrid best{4, 8};
+    uint64_t best_waves = ~0ull;
+    for (uint32_t nw : {4u, 6u, 8u}) {
+        const uint64_t busiest = ((waves + nw - 1) / nw + cus - 1) / cus * nw;
+        if (busiest <= best_waves) best.nw = nw, best_waves = busiest;
     }
     return best;
+}
+
+template <class Kern>
+static hipError_t lds_limit(Kern kern, uint32_t lds) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    return hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
 template <class QT, int MODE>
 static hipError_t gemv_dispatch(const uint8_t *w, uint64_t rows, uint64_t cols, const float *xf, const uint8_t *xq,
                                 float *y, hipStream_t st) {
-    const uint32_t items = (uint32_t)(cols / 256) * QT::IPB;
-    const uint32_t S = lanes_per_row(items);
-    const uint32_t ipl = items / S;
-    const uint64_t rb = cols / 256 * QT::BB;
-    const uint32_t lds = MODE == 0 ? actf_bytes((uint32_t)cols) : act_bytes((uint32_t)cols);
     const int cus = device_cu_count();
-    const uint32_t slots = 64 / S;
-    auto go = [&](auto kern, int rps, int nw) -> hipError_t {
-        const uint64_t rows_iter = (uint64_t)nw * slots * rps;
-        uint64_t iters = (rows + rows_iter - 1) / rows_iter;
-        const uint64_t cap = 8ull * cus;
+    const GemvShape sh = gemv_shape<QT>(rows, cols, (uint64_t)cus);
+    const uint64_t rb = cols / 256 * QT::BB;
+    const uint32_t lds = XLds<QT, MODE>::bytes((uint32_t)(cols / 256) * QT::IPB);
+    return with_n<gemv_nmax<QT>()>(sh.N, [&](auto n) -> hipError_t {
+        constexpr int N = decltype(n)::value, RPS = gemv_rps<QT>(N);
+        const uint32_t rows_per_wave = 64 / sh.S * RPS;
+        const uint64_t waves = (rows + rows_per_wave - 1) / rows_per_wave;
+        const GemvGrid gg = gemv_grid(waves, cols, cus);
+        const uint64_t iters = (waves + gg.nw - 1) / gg.nw, cap = (uint64_t)gg.cap * cus;
         const uint32_t grid = (uint32_t)(iters < cap ? iters : cap);
-        if (lds > 64 * 1024) {
-            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, st, w, (uint32_t)rows, (uint32_t)cols, rb,
-                           (uint32_t)ilog2(S), xf, xq, y);
+        auto kern = k_gemv<QT, N, RPS, MODE>;
+        const hipError_t e = lds_limit(kern, lds);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * gg.nw), lds, st, w, (uint32_t)rows, (uint32_t)cols, rb,
+                           (uint32_t)ilog2(sh.S), xf, xq, y);
         return hipGetLastError();
-    };
-    constexpr bool Q4 = QT::TYPE == T_Q4_K;
-    auto waves = [&](int rps) { return gemv_waves(rows, slots * rps, cus); };
-    switch (ipl) {
-        case 1:
-            if constexpr (Q4) {
-                switch (waves(4)) {
-                    case 6: return go(k_gemv<QT, 1, 4, MODE, 6>, 4, 6);
-                    case 8: return go(k_gemv<QT, 1, 4, MODE, 8>, 4, 8);
-                    default: return go(k_gemv<QT, 1, 4, MODE>, 4, 4);
-                }
-            } else {
-                return go(k_gemv<QT, 1, 2, MODE>, 2, 4);
-            }
-        case 2: return Q4 ? go(k_gemv<QT, 2, 2, MODE>, 2, 4) : go(k_gemv<QT, 2, 1, MODE>, 1, 4);
-        case 3: return go(k_gemv<QT, 3, 1, MODE>, 1, 4);
-        default: return go(k_gemv<QT, 0, 1, MODE>, 1, 4);
-    }
+    });
 }
 
-// Rows per workgroup pass of the unrolled instantiations (the same choice
-// gemv_dispatch makes; the generic path takes one row per lane slot).
-static int gemv_rps(uint32_t type, uint32_t ipl) {
-    if (type == T_Q4_K) return ipl == 1 ? 4 : (ipl == 2 ? 2 : 1);
-    return ipl == 1 ? 2 : 1;
-}
-
-hipError_t launch_gemv_multi(int n, const uint32_t *types, const uint8_t *const *ws, const uint64_t *rows,
-                             uint64_t cols, const float *x, float *const *ys, int mode, hipStream_t st) {
-    GemvMultiArgs g{};
-    const uint32_t items4 = (uint32_t)(cols / 256) * Q4K::IPB, items6 = (uint32_t)(cols / 256) * Q6K::IPB;
-    const uint32_t s4 = lanes_per_row(items4), s6 = lanes_per_row(items6);
-    const uint32_t ipl4 = items4 / s4, ipl6 = items6 / s6;
-    // The unrolled pairs that one column count gives (cols 256..2048, 4096,
-    // 6144); any other pair runs the generic item loop for both types.
-    int sel = 0;   // 0 generic, 1 (1,1), 2 (2,1), 3 (3,3)
-    if (ipl4 == 1 && ipl6 == 1) sel = 1;
-    else if (ipl4 == 2 && ipl6 == 1) sel = 2;
-    else if (ipl4 == 3 && ipl6 == 3) sel = 3;
+template <int MODE>
+static hipError_t gemv_multi_dispatch(GemvMultiArgs &g, int n, const uint64_t *rows, hipStream_t st) {
+    // N by the row length alone (one kernel for all the matrices); S per
+    // matrix as the single GEMV takes it: a row's bits depend on S only
+    const GemvShape s4 = gemv_shape<Q4K>(0, g.cols, 1), s6 = gemv_shape<Q6K>(0, g.cols, 1);
+    const uint32_t nb = g.cols / 256, cus = (uint32_t)device_cu_count();
     uint64_t iters[GEMV_MULTI_MAX] = {0}, total = 0;
+    uint32_t lds = 0;
     for (int i = 0; i < n; i++) {
-        const uint32_t ipl = types[i] == T_Q4_K ? ipl4 : ipl6;
-        const uint32_t S = types[i] == T_Q4_K ? s4 : s6;
-        const uint64_t rows_iter = 4ull * (64 / S) * (sel ? gemv_rps(types[i], ipl) : 1);
-        iters[i] = (rows[i] + rows_iter - 1) / rows_iter;
+        const bool q4 = g.type[i] == T_Q4_K;
+        const uint32_t S = q4 ? gemv_shape<Q4K>(rows[i], g.cols, cus).S : gemv_shape<Q6K>(rows[i], g.cols, cus).S;
+        const uint32_t rows_per_wave = 64 / S * (q4 ? gemv_rps<Q4K>(s4.N) : gemv_rps<Q6K>(s6.N));
+        g.log2s[i] = (uint32_t)ilog2(S);
+        iters[i] = (rows[i] + rows_per_wave - 1) / rows_per_wave;
         total += iters[i];
+        const uint32_t b = q4 ? XLds<Q4K, MODE>::bytes(nb * Q4K::IPB) : XLds<Q6K, MODE>::bytes(nb * Q6K::IPB);
+        if (rows[i] && b > lds) lds = b;
     }
     if (!total) return hipSuccess;
-    const uint64_t cap = 8ull * device_cu_count();
+    // The matrices' workgroups differ in work, and small ones even that out:
+    // q, k and v of 4096 columns take 6.6 us in 4 waves, 8.3 in 6, 7.6 in 8.
+    GemvGrid gg{4, 8};
+    if (total > 16ull * cus) gg = gemv_grid(total, g.cols, cus);
+    total = 0;
+    for (int i = 0; i < n; i++) {   // waves -> workgroups
+        iters[i] = (iters[i] + gg.nw - 1) / gg.nw;
+        total += iters[i];
+    }
+    const uint64_t cap = (uint64_t)gg.cap * cus;
     uint32_t end = 0;
     for (int i = 0; i < GEMV_MULTI_MAX; i++) {
         if (i < n) {
@@ -386,40 +550,37 @@ hipError_t launch_gemv_multi(int n, const uint32_t *types, const uint8_t *const 
                 if (!wg) wg = 1;
             }
             end += (uint32_t)wg;
-            g.w[i] = ws[i];
-            g.y[i] = ys[i];
-            g.rows[i] = (uint32_t)rows[i];
-            g.type[i] = types[i];
         }
         g.end[i] = end;   // past n: the total, so no workgroup maps there
     }
+    return with_n<gemv_nmax<Q4K>()>(s4.N, [&](auto n4) {
+        return with_n<gemv_nmax<Q6K>()>(s6.N, [&](auto n6) -> hipError_t {
+            constexpr int N4 = decltype(n4)::value, N6 = decltype(n6)::value;
+            if constexpr (!gemv_pair(N4, N6)) {
+                return hipErrorInvalidValue;
+            } else {
+                auto kern = k_gemv_multi<N4, N6, MODE>;
+                const hipError_t e = lds_limit(kern, lds);
+                if (e != hipSuccess) return e;
+                hipLaunchKernelGGL(kern, dim3(end), dim3(64 * gg.nw), lds, st, g);
+                return hipGetLastError();
+            }
+        });
+    });
+}
+
+hipError_t launch_gemv_multi(int n, const uint32_t *types, const uint8_t *const *ws, const uint64_t *rows,
+                             uint64_t cols, const float *x, float *const *ys, int mode, hipStream_t st) {
+    GemvMultiArgs g{};
+    for (int i = 0; i < n; i++) {
+        g.w[i] = ws[i];
+        g.y[i] = ys[i];
+        g.rows[i] = (uint32_t)rows[i];
+        g.type[i] = types[i];
+    }
     g.cols = (uint32_t)cols;
-    g.log2s4 = (uint32_t)ilog2(s4);
-    g.log2s6 = (uint32_t)ilog2(s6);
     g.x = x;
-    const uint32_t lds = mode == 0 ? actf_bytes((uint32_t)cols) : act_bytes((uint32_t)cols);
-    auto go = [&](auto kern) -> hipError_t {
-        if (lds > 64 * 1024) {
-            hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(kern, dim3(end), dim3(256), lds, st, g);
-        return hipGetLastError();
-    };
-    if (mode == 0) {
-        switch (sel) {
-            case 1: return go(k_gemv_multi<1, 4, 1, 2, 0>);
-            case 2: return go(k_gemv_multi<2, 2, 1, 2, 0>);
-            case 3: return go(k_gemv_multi<3, 1, 3, 1, 0>);
-            default: return go(k_gemv_multi<0, 1, 0, 1, 0>);
-        }
-    }
-    switch (sel) {
-        case 1: return go(k_gemv_multi<1, 4, 1, 2, 2>);
-        case 2: return go(k_gemv_multi<2, 2, 1, 2, 2>);
-        case 3: return go(k_gemv_multi<3, 1, 3, 1, 2>);
-        default: return go(k_gemv_multi<0, 1, 0, 1, 2>);
-    }
+    return mode == 0 ? gemv_multi_dispatch<0>(g, n, rows, st) : gemv_multi_dispatch<2>(g, n, rows, st);
 }
 
 hipError_t launch_gemv(uint32_t type, const uint8_t *w, uint64_t rows, uint64_t cols, const float *xf,

@@ -41,7 +41,8 @@ struct GemvMultiArgs {
     uint32_t rows[GEMV_MULTI_MAX];
     uint32_t type[GEMV_MULTI_MAX];
     uint32_t end[GEMV_MULTI_MAX];   // cumulative workgroup counts
-    uint32_t cols, log2s4, log2s6;
+    uint32_t log2s[GEMV_MULTI_MAX]; // lanes per row
+    uint32_t cols;
     const float *x;
 };
 hipError_t launch_gemv_multi(int n, const uint32_t *types, const uint8_t *const *ws, const uint64_t *rows,
