@@ -17,6 +17,8 @@
 
 namespace kq {
 
+constexpr int32_t NONE = 0x7FFFFFFF;
+
 struct Best {
     float v;
     int32_t i;
@@ -24,15 +26,28 @@ struct Best {
 __device__ __forceinline__ Best better(Best a, Best b) {
     return (b.v > a.v || (b.v == a.v && b.i < a.i)) ? b : a;
 }
+// On the VALU (DPP, permlane swaps): the wave's largest value, then the
+// lowest index that holds it. Values are never NaN; -0 and +0 compare equal.
 __device__ __forceinline__ Best wave_best(Best b) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        Best p;
-        p.v = __shfl_xor(b.v, o, WAVE);
-        p.i = __shfl_xor(b.i, o, WAVE);
-        b = better(b, p);
-    }
-    return b;
+    float m = b.v;
+    m = fmaxf(m, dpp_f<DPP_XOR1>(m));
+    m = fmaxf(m, dpp_f<DPP_XOR2>(m));
+    m = fmaxf(m, dpp_f<DPP_HALF_MIRROR>(m));
+    m = fmaxf(m, dpp_f<DPP_MIRROR>(m));
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    m = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+    m = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    int i = b.v == m ? b.i : NONE;
+    i = min(i, dpp_i<DPP_XOR1>(i));
+    i = min(i, dpp_i<DPP_XOR2>(i));
+    i = min(i, dpp_i<DPP_HALF_MIRROR>(i));
+    i = min(i, dpp_i<DPP_MIRROR>(i));
+    r = __builtin_amdgcn_permlane16_swap((uint32_t)i, (uint32_t)i, false, false);
+    i = min((int)r[0], (int)r[1]);
+    r = __builtin_amdgcn_permlane32_swap((uint32_t)i, (uint32_t)i, false, false);
+    i = min((int)r[0], (int)r[1]);
+    return Best{m, i};
 }
 __device__ __forceinline__ Best block_best(Best b) {
     __shared__ Best part[4];
@@ -45,8 +60,8 @@ __device__ __forceinline__ Best block_best(Best b) {
     return b;
 }
 
-constexpr int32_t NONE = 0x7FFFFFFF;
 constexpr uint32_t ARGMAX_PARTS = 256;
+constexpr uint32_t ARGMAX_U = 4;
 constexpr uint32_t ARGMAX_COUNT = 2 * ARGMAX_PARTS;   // the count word, after the partials
 
 __device__ __forceinline__ uint64_t pack(Best b) { return ((uint64_t)(uint32_t)b.i << 32) | __float_as_uint(b.v); }
@@ -57,9 +72,18 @@ __global__ void __launch_bounds__(256) k_argmax(const float *__restrict__ x, uin
                                                 int32_t *out) {
     __shared__ uint32_t last;
     Best b{-FLT_MAX, NONE};
-    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < n; t += gridDim.x * 256) {
-        const float v = x[t];
-        if (v > b.v) b = Best{v, (int32_t)t};   // ascending t per thread: strict > keeps the first
+    // ascending t per thread: strict > keeps the first. ARGMAX_U loads in flight
+    // per round (positions past n load x[n - 1] and are dropped).
+    for (uint32_t t0 = blockIdx.x * 256 + threadIdx.x, st = gridDim.x * 256; t0 < n;) {
+        float v[ARGMAX_U];
+        const uint32_t left = (n - 1 - t0) / st;   // positions t0 + st k, k <= left, are in range
+#pragma unroll
+        for (uint32_t k = 0; k < ARGMAX_U; k++) v[k] = x[k <= left ? t0 + st * k : n - 1];
+#pragma unroll
+        for (uint32_t k = 0; k < ARGMAX_U; k++)
+            if (k <= left && v[k] > b.v) b = Best{v[k], (int32_t)(t0 + st * k)};
+        if (left < ARGMAX_U) break;
+        t0 += st * ARGMAX_U;
     }
     b = block_best(b);
     if (threadIdx.x == 0) {
@@ -82,7 +106,7 @@ __global__ void __launch_bounds__(256) k_argmax(const float *__restrict__ x, uin
 uint32_t argmax_scratch_bytes() { return 4 * (ARGMAX_COUNT + 1); }
 
 hipError_t launch_argmax(const float *x, uint32_t n, void *scratch, int32_t *out, hipStream_t s) {
-    uint32_t g = (n + 2047) / 2048;
+    uint32_t g = (n + 256 * ARGMAX_U - 1) / (256 * ARGMAX_U);
     if (g < 1) g = 1;
     if (g > ARGMAX_PARTS) g = ARGMAX_PARTS;
     hipLaunchKernelGGL(k_argmax, dim3(g), dim3(256), 0, s, x, n, (uint32_t *)scratch, out);
