@@ -126,6 +126,10 @@ struct MoeArgs {
     // launcher from xcd_local(); callers leave it 0)
     uint32_t hloc;
 };
+// Kernel B for rows of more than four blocks (kq_moe_down.hip), after kernel A
+// has written h and the routing; hipErrorNotSupported when the shape is
+// kernel B's own (shorter rows, or h past the LDS in its layout).
+hipError_t launch_moe_down_wide(const MoeArgs &a, uint32_t n_slots, hipStream_t s);
 bool moe_shape_supported(uint32_t gate_type, uint32_t down_type, uint32_t hidden, uint32_t ffn);
 // Dynamic LDS (bytes) of the largest workgroup a layer of this shape launches:
 // kernel A, kernel B (n_slots * (ffn + ffn/8 + ffn/4) for the staged h, plus

@@ -1420,11 +1420,11 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
     const bool routed = (int)sl < a.n_sel;
     const uint8_t *db = routed ? a.down + (uint64_t)sid * a.hidden * rbd : a.down_sh;
     const uint8_t *rp = db + (uint64_t)(row0 + r) * rbd;
-    typename QD::Raw raw[IPL > 0 ? IPL : 1];
+    typename QD::RawQ raw[IPL > 0 ? IPL : 1];   // (the lanes of a quad hold one block's items)
     if constexpr (IPL > 0) {
 #pragma unroll
         for (int i = 0; i < IPL; i++)   // clamped: a block past the row is loaded and dropped
-            raw[i] = QD::load(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
+            raw[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
     }
     stage_h(lds + L.hacts, a.ffn, ntask, 0, nt, hv);
     for (uint32_t first = HT * nt; first < ntask; first += HT * nt) {
@@ -1439,7 +1439,7 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
 #pragma unroll
             for (int i = 0; i < IPL; i++) {
                 const uint32_t b = sub + P * i;
-                const float v = QD::dot_q8(raw[i], (int)item, act, min(b, nbk - 1));
+                const float v = QD::dot_q8(QD::full(raw[i]), (int)item, act, min(b, nbk - 1));
                 x += b < nbk ? v : 0.0f;
             }
         } else {
@@ -1667,18 +1667,22 @@ __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
     const uint32_t r = min(ls, nrows - 1);   // idle lane-slots load a real row and drop it
     const uint8_t *db = ex >= a.n_expert ? a.down_sh : a.down + (uint64_t)ex * a.hidden * rbd;
     const uint8_t *rp = db + (uint64_t)(row0 + r) * rbd;
-    typename QD::Raw raw[IPL > 0 ? IPL : 1];
+    typename QD::RawQ rawq[IPL > 0 ? IPL : 1];   // (the lanes of a quad hold one block's items)
     if constexpr (IPL > 0) {
 #pragma unroll
-        for (int i = 0; i < IPL; i++) raw[i] = QD::load(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
+        for (int i = 0; i < IPL; i++) rawq[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
     }
     const uint64_t hstride = (uint64_t)(a.ffn / 32) * 36;
     stage_rows_q8(lds, a.ffn, cnt, [&](uint32_t g) { return a.hq8 + (uint64_t)pairs[g] * hstride; });
     // the quants are unpacked once for all pairs
+    typename QD::Raw raw[IPL > 0 ? IPL : 1];
     typename QD::Unp unp[IPL > 0 ? IPL : 1];
     if constexpr (IPL > 0) {
 #pragma unroll
-        for (int i = 0; i < IPL; i++) unp[i] = QD::unpack(raw[i]);
+        for (int i = 0; i < IPL; i++) {
+            raw[i] = QD::full(rawq[i]);
+            unp[i] = QD::unpack(raw[i]);
+        }
     }
     __syncthreads();
     const uint32_t ab = act_bytes(a.ffn);
@@ -3111,6 +3115,15 @@ static hipError_t go_b_any(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, 
     return go_b<QD, 0, 1>(a, n_slots, pl, s);
 }
 static hipError_t go_b_run(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, hipStream_t s) {
+    // What would run the runtime block loop, and the whole-wave rows of two
+    // and more slots, have their own kernel (two slots of 14336, Q6_K: 25.8 ->
+    // 22.2 us; six of 9728, Q4_K: 39.8 -> 18.0; ten of 4096, Q4_K: 38.1 ->
+    // 14.2). One slot (a dense FFN) has one pair per wave there and gains
+    // nothing: 10.9 us here at 12288, 11.4 there.
+    if (pl.key == 0 || (pl.key >= 16 * 8 && n_slots > 1)) {
+        const hipError_t e = launch_moe_down_wide(a, n_slots, s);
+        if (e != hipErrorNotSupported) return e;
+    }
     return a.down_type == T_Q6_K ? go_b_any<Q6K>(a, n_slots, pl, s) : go_b_any<Q4K>(a, n_slots, pl, s);
 }
 
