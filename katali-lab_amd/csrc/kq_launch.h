@@ -77,6 +77,8 @@ hipError_t launch_add_rmsnorm(float *x, const float *delta, float scale, const f
                               float *out, hipStream_t s);
 hipError_t launch_argmax(const float *x, uint32_t n, void *scratch, int32_t *out, hipStream_t s);
 
+constexpr uint32_t GRP_REC = 12;   // ints of a small-entry record of the batched layer
+
 // MoE layer (two launches). Types: gate/up Q4_K; down Q4_K or Q6_K.
 struct MoeArgs {
     const uint8_t *gate, *up, *down;          // stacked [n_expert][rows][row_bytes]
@@ -102,13 +104,12 @@ struct MoeArgs {
     int32_t *err;            // error word (bit 1: expert id out of range, bit 2: fused-layer wait expired)
     uint32_t *fsync;         // fused layer's exchange (layout at fsync_words())
     // Batched layer (several tokens): a pair p = t * bS + r is token t's rank
-    // r (r == n_sel: the shared expert). bslot holds *bcount {expert, first,
-    // count} entries whose pairs are border[first .. first + count); x comes
-    // from the q8_1 rows xq + t * xq_stride, h goes to hq8 row p and the
-    // pair's unweighted down output to yp + p * hidden.
+    // r (r == n_sel: the shared expert). bslot holds *bcount entry records of
+    // GRP_REC ints {expert, count, 0, 0, 8 pairs}, slots past count holding
+    // pair 0; x comes from the q8_1 rows xq + t * xq_stride, h goes to hq8 row
+    // p and the pair's unweighted down output to yp + p * hidden.
     const int32_t *bslot;
     const int32_t *bcount;
-    const int32_t *border;
     uint32_t bS;
     uint64_t xq_stride;
     float *yp;

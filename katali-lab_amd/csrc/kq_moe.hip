@@ -328,8 +328,20 @@ __device__ __forceinline__ float q4k_term(const uint4 &q, const float4 &sc, cons
     Q4K::isums_x(q, x.xl, x.xh, slo, shi);
     return q4k_term_from(slo, shi, sc, x.xsum);
 }
-// q4k_term with the nibbles unpacked beforehand (the same sums and float ops)
-__device__ __forceinline__ float q4k_term_u(const Q4K::Unp &u, const float4 &sc, const XSlice &x) {
+// The same with the lane's own sub-block's {d * sc, dmin * m} and q8_1 scale
+// d8 apart (A = s.x * d8, B = s.y * d8: the products a scale table folds)
+__device__ __forceinline__ float q4k_term_own(int slo, int shi, float2 s, float d8, float xsum) {
+    const bool hh = threadIdx.x & 1;
+    const int isum = (hh ? shi : slo) + dpp_i<DPP_XOR1>(hh ? slo : shi);
+    return fmaf(s.x * d8, (float)isum, -((s.y * d8) * xsum));
+}
+__device__ __forceinline__ float q4k_term(const uint4 &q, float2 s, float d8, const XSlice &x) {
+    int slo, shi;
+    Q4K::isums_x(q, x.xl, x.xh, slo, shi);
+    return q4k_term_own(slo, shi, s, d8, x.xsum);
+}
+// ... with the nibbles unpacked beforehand (the same sums and float ops)
+__device__ __forceinline__ float q4k_term_u(const Q4K::Unp &u, float2 s, float d8, const XSlice &x) {
     int slo = dot4(u.lo.x, x.xl.x, 0);
     slo = dot4(u.lo.y, x.xl.y, slo);
     slo = dot4(u.lo.z, x.xl.z, slo);
@@ -338,7 +350,7 @@ __device__ __forceinline__ float q4k_term_u(const Q4K::Unp &u, const float4 &sc,
     shi = dot4(u.hi.y, x.xh.y, shi);
     shi = dot4(u.hi.z, x.xh.z, shi);
     shi = dot4(u.hi.w, x.xh.w, shi);
-    return q4k_term_from(slo, shi, sc, x.xsum);
+    return q4k_term_own(slo, shi, s, d8, x.xsum);
 }
 
 // Rows of sub-block terms summed pairwise over the lanes. Chunk k of a lane
@@ -1470,34 +1482,57 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
 
 // ---------------------------------------------------------------------------
 // Grouped batch mode: the GEMV path of the batched layer. An entry is up to
-// GRP_MAX (token, rank) pairs routed to one expert, listed as {expert,
-// first, count} (a.bslot, *a.bcount entries) with the pairs at
-// a.border[first ..]. A workgroup reads its weight rows once and dots them
-// with every pair of the entry, whose activations are staged in LDS. The
-// item mapping, scale products, reductions and h quantization are those of
-// kernels A and B, so a pair's h and down output are bit-identical to the
-// single-token layer's.
+// GRP_MAX (token, rank) pairs routed to one expert, listed as a record of
+// GRP_REC ints (a.bslot, *a.bcount entries). A workgroup reads its weight rows
+// once and dots them with every pair of the entry, whose activations are
+// staged in LDS. The item mapping, scale products, reductions and h
+// quantization are those of kernels A and B, so a pair's h and down output are
+// bit-identical to the single-token layer's.
+//
+// Order of a workgroup's loads: its record, count and pairs at once; then the
+// pairs' activations (L2), then the weights (HBM): loads return in order, so
+// activations issued behind the weights, after a load of their pairs, came two
+// round trips after the last weight.
 // ---------------------------------------------------------------------------
 constexpr uint32_t GRP_MAX = 8;
 
-// Stage n rows of K q8_1 values (row g read from src_of(g)) into LDS
-// activations at base + g * act_bytes(K), one 16-byte half block per task.
-template <class SrcOf>
-__device__ __forceinline__ void stage_rows_q8(uint8_t *base, uint32_t K, uint32_t n, SrcOf src_of) {
-    const uint32_t nblk = K / 32, ab = act_bytes(K), ntask = n * nblk * 2;
-    for (uint32_t t = threadIdx.x; t < ntask; t += blockDim.x) {
-        const uint32_t g = t / (2 * nblk), r = t % (2 * nblk), kb = r >> 1, half = r & 1;
-        const uint8_t *b = src_of(g) + (uint64_t)kb * 36;
-        const uint4 q = ld16(b + 4 + 16 * half);
-        const Act act = act_carve(base + g * ab, K);
-        *(uint4 *)(act.qs + 32 * kb + 16 * half) = q;
-        int sum = dot4(q.x, 0x01010101u, 0);
-        sum = dot4(q.y, 0x01010101u, sum);
-        sum = dot4(q.z, 0x01010101u, sum);
-        sum = dot4(q.w, 0x01010101u, sum);
-        act.qs16[2 * kb + half] = sum;
-        if (half == 0) act.d8[kb] = h2f(ld_u16(b));
-    }
+struct GrpEntry {
+    uint32_t ex, cnt;   // uniform
+    uint32_t pair;      // lane l: pair l % GRP_MAX (pair 0 past the count)
+};
+// The record of entry ei; cnt 0 when the list has no such entry (the record is
+// inside the list's memory all the same).
+__device__ __forceinline__ GrpEntry grp_entry(const MoeArgs &a, uint32_t ei) {
+    const int32_t *rec = a.bslot + (uint64_t)GRP_REC * ei;
+    const int32_t n = *a.bcount, ex = rec[0], cnt = rec[1];
+    GrpEntry e;
+    e.pair = (uint32_t)rec[4 + (threadIdx.x & (GRP_MAX - 1))];
+    e.ex = (uint32_t)__builtin_amdgcn_readfirstlane(ex);
+    e.cnt = ei < (uint32_t)__builtin_amdgcn_readfirstlane(n) ? (uint32_t)__builtin_amdgcn_readfirstlane(cnt) : 0u;
+    return e;
+}
+
+// One 16-byte half block of a pair's q8_1 row: half block r of pair g
+struct GrpX {
+    uint4 q;
+    uint32_t d;
+};
+__device__ __forceinline__ GrpX grp_load(const uint8_t *row, uint32_t r) {
+    const uint8_t *b = row + (uint64_t)(r >> 1) * 36;
+    GrpX v;
+    v.q = ld16(b + 4 + 16 * (r & 1));
+    v.d = ld_u16(b);
+    return v;
+}
+__device__ __forceinline__ void grp_put(uint8_t *base, uint32_t K, uint32_t g, uint32_t r, const GrpX &v) {
+    const Act act = act_carve(base + g * act_bytes(K), K);
+    *(uint4 *)(act.qs + 16 * r) = v.q;
+    int sum = dot4(v.q.x, 0x01010101u, 0);
+    sum = dot4(v.q.y, 0x01010101u, sum);
+    sum = dot4(v.q.z, 0x01010101u, sum);
+    sum = dot4(v.q.w, 0x01010101u, sum);
+    act.qs16[r] = sum;
+    if ((r & 1) == 0) act.d8[r >> 1] = h2f(v.d);
 }
 
 struct LdsG {
@@ -1525,10 +1560,9 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t nblk = a.ffn / 32;
     const uint32_t ei = blockIdx.x / nblk, jb = blockIdx.x % nblk;
-    if (ei >= (uint32_t)*a.bcount) return;   // whole workgroup, before any barrier
-    const int32_t *ent = a.bslot + 3 * ei;
-    const uint32_t ex = (uint32_t)ent[0], cnt = (uint32_t)ent[2];
-    const int32_t *pairs = a.border + ent[1];
+    const GrpEntry ent = grp_entry(a, ei);
+    const uint32_t ex = ent.ex, cnt = ent.cnt;
+    if (cnt == 0) return;   // whole workgroup, before any barrier
     const uint64_t rb = NB * 144;
     const bool shared = ex >= a.n_expert;   // the grouping gives the shared expert id n_expert
     const uint8_t *gb = shared ? a.gate_sh : a.gate + (uint64_t)ex * a.ffn * rb;
@@ -1547,7 +1581,19 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
         }
         return row_ptr(RW * wave + r) + (it / 8) * 144 + 16 + 16 * (it % 8);
     };
-    // the weights (HBM) first, then the entry's activations (L2)
+    // the entry's activations (L2) first, then the weights (HBM)
+    constexpr uint32_t XPR = 16 * NB;                                  // half blocks per row
+    constexpr int XT = (GRP_MAX * XPR + A_THREADS - 1) / A_THREADS;    // per thread, at most
+    const uint32_t tok = ent.pair / a.bS;
+    GrpX xv[XT];
+#pragma unroll
+    for (int i = 0; i < XT; i++) {
+        const uint32_t t = tid + A_THREADS * i;
+        const uint32_t st = (uint32_t)__shfl((int)tok, (int)min(t / XPR, cnt - 1), WAVE);   // past the entry: its last row
+        xv[i] = grp_load(a.xq + (uint64_t)st * a.xq_stride, t % XPR);
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     uint4 hv[HPL];
 #pragma unroll
     for (int i = 0; i < HPL; i++) {
@@ -1557,12 +1603,17 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
     uint4 q[LPG];
 #pragma unroll
     for (int k = 0; k < LPG; k++) q[k] = ld16(chunk(k));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);   // every weight load is out before the activations are staged
     const uint32_t ab = act_bytes(a.hidden);
-    stage_rows_q8(lds + L.xact, a.hidden, cnt,
-                  [&](uint32_t g) { return a.xq + (uint64_t)((uint32_t)pairs[g] / a.bS) * a.xq_stride; });
-    // the wave's headers -> {d*sc, d*sc', dmin*m, dmin*m'} per group (x's
-    // q8_1 scales are applied per pair below, in kernel A's order)
-    float4 *scl = (float4 *)(lds + L.scl) + 4 * WH * wave;
+#pragma unroll
+    for (int i = 0; i < XT; i++) {
+        const uint32_t t = tid + A_THREADS * i;
+        if (t < cnt * XPR) grp_put(lds + L.xact, a.hidden, t / XPR, t % XPR, xv[i]);
+    }
+    // the wave's headers -> {d*sc, dmin*m} per sub-block (x's q8_1 scales are
+    // applied per pair below, in kernel A's order)
+    float2 *scl = (float2 *)(lds + L.scl) + 8 * WH * wave;
 #pragma unroll
     for (int i = 0; i < HPL; i++) {
         const uint32_t h = lane + 64 * i;
@@ -1573,7 +1624,7 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
             for (int g = 0; g < 4; g++) {
                 float ds0, ds1, dm0, dm1;
                 Q4K::scales(raw, g, ds0, ds1, dm0, dm1);
-                scl[4 * h + g] = make_float4(ds0, ds1, dm0, dm1);
+                *(float4 *)(scl + 8 * h + 2 * g) = make_float4(ds0, dm0, ds1, dm1);
             }
         }
     }
@@ -1590,41 +1641,42 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
     }
     __syncthreads();   // activations staged; the scale table is wave-private
 
+    // a lane's item it ends with the sum of sub-block it of its row: that
+    // sub-block's scales, held for all pairs (read per pair, for both
+    // sub-blocks of the group, they were 8 LDS reads and 32 products of 190
+    // instructions per pair)
+    float2 sc[LPG];
+#pragma unroll
+    for (int k = 0; k < LPG; k++)
+        sc[k] = scl[ITEMS >= 64 ? ITEMS * (k / M) + 64 * (k % M) + lane
+                                : ITEMS * (lane / ITEMS + k * (64 / ITEMS)) + lane % ITEMS];
     float *gu = (float *)(lds + L.gu);
     for (uint32_t g = 0; g < cnt; g++) {
         const Act xa = act_carve(lds + L.xact + g * ab, a.hidden);
         if constexpr (ITEMS >= 64) {
             XSlice xs[M];
-            float2 d8[M];
+            float d8[M];
 #pragma unroll
             for (int m = 0; m < M; m++) {
-                const uint32_t it = 64 * m + lane, k8 = 8 * (it / 8) + 2 * ((it % 8) >> 1);
-                xs[m] = x_slice(xa, it);
-                d8[m] = make_float2(xa.d8[k8], xa.d8[k8 + 1]);
+                xs[m] = x_slice(xa, 64 * m + lane);
+                d8[m] = xa.d8[64 * m + lane];
             }
             float acc[LPG];   // virtual row k: sub-block 64 * (k % M) + lane of row k / M
 #pragma unroll
             for (int k = 0; k < LPG; k++) {
-                const uint32_t it = 64 * (k % M) + lane;
-                const uint32_t row = k / M;
-                const float4 s0 = scl[4 * (row * NB + it / 8) + (it % 8) / 2];
-                const float2 dd = d8[k % M];
-                const float4 sc = make_float4(s0.x * dd.x, s0.y * dd.y, s0.z * dd.x, s0.w * dd.y);
-                if constexpr (UNP) acc[k] = q4k_term_u(qu[k], sc, xs[k % M]);
-                else acc[k] = q4k_term(q[k], sc, xs[k % M]);
+                if constexpr (UNP) acc[k] = q4k_term_u(qu[k], sc[k], d8[k % M], xs[k % M]);
+                else acc[k] = q4k_term(q[k], sc[k], d8[k % M], xs[k % M]);
             }
             const float v = pw_rows<LPG, M>(acc);
             if (lane < (uint32_t)RW) gu[64 * g + RW * wave + pw_rows_row<LPG, M>(lane)] = v;
         } else {
-            const uint32_t it = lane % ITEMS, k8 = 8 * (it / 8) + 2 * ((it % 8) >> 1);
+            const uint32_t it = lane % ITEMS;
             const XSlice xs = x_slice(xa, it);
-            const float2 dd = make_float2(xa.d8[k8], xa.d8[k8 + 1]);
+            const float d8 = xa.d8[it];
 #pragma unroll
             for (int k = 0; k < LPG; k++) {
                 const uint32_t row = lane / ITEMS + k * (64 / ITEMS);
-                const float4 s0 = scl[4 * (row * NB + it / 8) + (it % 8) / 2];
-                const float4 sc = make_float4(s0.x * dd.x, s0.y * dd.y, s0.z * dd.x, s0.w * dd.y);
-                const float v = group_sum<ITEMS>(UNP ? q4k_term_u(qu[k], sc, xs) : q4k_term(q[k], sc, xs));
+                const float v = group_sum<ITEMS>(UNP ? q4k_term_u(qu[k], sc[k], d8, xs) : q4k_term(q[k], sc[k], d8, xs));
                 if (it == 0) gu[64 * g + RW * wave + row] = v;
             }
         }
@@ -1639,7 +1691,8 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
         const float id = d != 0.0f ? 1.0f / d : 0.0f;
         const int qv = (int)roundf(h * id);
         const int total = sum32(qv);
-        uint8_t *blk = a.hq8 + ((uint64_t)pairs[g] * nblk + jb) * 36;
+        const uint32_t pair = (uint32_t)__builtin_amdgcn_readlane((int)ent.pair, (int)g);
+        uint8_t *blk = a.hq8 + ((uint64_t)pair * nblk + jb) * 36;
         if (lane < 32) blk[4 + lane] = (uint8_t)(qv & 255);
         if (lane == 0) *(uint32_t *)blk = f2h_rne(d) | (f2h_rne((float)total * d) << 16);
     }
@@ -1652,10 +1705,31 @@ template <class QD, int IPL, int P>
 __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t tid = threadIdx.x;
-    if (blockIdx.y >= (uint32_t)*a.bcount) return;   // whole workgroup, before any barrier
-    const int32_t *ent = a.bslot + 3 * blockIdx.y;
-    const uint32_t ex = (uint32_t)ent[0], cnt = (uint32_t)ent[2];
-    const int32_t *pairs = a.border + ent[1];
+    const GrpEntry ent = grp_entry(a, blockIdx.y);
+    const uint32_t ex = ent.ex, cnt = ent.cnt;
+    if (cnt == 0) return;   // whole workgroup, before any barrier
+    // h first (L2), as the gate/up kernel's activations: up to HT tasks per
+    // thread ahead of the weights (all of them up to 2048-wide rows), the
+    // rest behind
+    constexpr int HT = P == 1 ? 2 : 4;
+    const uint64_t hstride = (uint64_t)(a.ffn / 32) * 36;
+    const uint32_t per = a.ffn / 16, ntask = cnt * per;
+    auto task = [&](uint32_t t, uint32_t &g, uint32_t &r) {   // half block r of pair g
+        g = 0;
+#pragma unroll
+        for (uint32_t k = 1; k < GRP_MAX; k++) g += t >= k * per ? 1u : 0u;
+        r = t - g * per;
+    };
+    auto h_load = [&](uint32_t t) {
+        uint32_t g, r;
+        task(t, g, r);
+        return grp_load(a.hq8 + (uint64_t)(uint32_t)__shfl((int)ent.pair, (int)g, WAVE) * hstride, r);
+    };
+    GrpX hv[HT];
+#pragma unroll
+    for (int i = 0; i < HT; i++) hv[i] = h_load(min(tid + 256 * i, ntask - 1));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     constexpr uint32_t S = QD::IPB * P;
     const uint32_t ls = tid / S, s = tid % S;
     const uint32_t item = s % QD::IPB, sub = s / QD::IPB;
@@ -1672,8 +1746,20 @@ __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
 #pragma unroll
         for (int i = 0; i < IPL; i++) rawq[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
     }
-    const uint64_t hstride = (uint64_t)(a.ffn / 32) * 36;
-    stage_rows_q8(lds, a.ffn, cnt, [&](uint32_t g) { return a.hq8 + (uint64_t)pairs[g] * hstride; });
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);   // every weight load is out before h is staged
+    auto h_put = [&](uint32_t t, const GrpX &v) {
+        uint32_t g, r;
+        task(t, g, r);
+        grp_put(lds, a.ffn, g, r, v);
+    };
+#pragma unroll
+    for (int i = 0; i < HT; i++)
+        if (tid + 256 * i < ntask) h_put(tid + 256 * i, hv[i]);
+    for (uint32_t t0 = 256 * HT; t0 < ntask; t0 += 256) {   // whole waves load (the lane exchange)
+        const GrpX v = h_load(min(tid + t0, ntask - 1));
+        if (tid + t0 < ntask) h_put(tid + t0, v);
+    }
     // the quants are unpacked once for all pairs
     typename QD::Raw raw[IPL > 0 ? IPL : 1];
     typename QD::Unp unp[IPL > 0 ? IPL : 1];
@@ -1700,7 +1786,8 @@ __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
             for (uint32_t b = sub; b < nbk; b += P) x += QD::dot_q8(QD::load(rp + b * QD::BB, (int)item), (int)item, act, b);
         }
         x = group_sum<S>(x);
-        if (active && s == 0) a.yp[(uint64_t)pairs[g] * a.hidden + row0 + ls] = x;
+        const uint32_t pair = (uint32_t)__builtin_amdgcn_readlane((int)ent.pair, (int)g);
+        if (active && s == 0) a.yp[(uint64_t)pair * a.hidden + row0 + ls] = x;
     }
 }
 
@@ -3293,7 +3380,7 @@ static hipError_t go_a_grp(const MoeArgs &a, uint32_t max_entries, hipStream_t s
 }
 
 hipError_t launch_moe_groups_gu(const MoeArgs &a, uint32_t max_entries, hipStream_t s) {
-    if (!a.bslot || !a.bcount || !a.border || max_entries == 0) return hipErrorInvalidValue;
+    if (!a.bslot || !a.bcount || max_entries == 0) return hipErrorInvalidValue;
     switch (a.hidden / 256) {
         case 1: return go_a_grp<1>(a, max_entries, s);
         case 2: return go_a_grp<2>(a, max_entries, s);
@@ -3347,7 +3434,7 @@ static hipError_t go_b_grp_any(const MoeArgs &a, uint32_t max_entries, hipStream
 }
 
 hipError_t launch_moe_groups_down(const MoeArgs &a, uint32_t max_entries, hipStream_t s) {
-    if (!a.bslot || !a.bcount || !a.border || !a.yp || max_entries == 0 || max_entries > 65535) return hipErrorInvalidValue;
+    if (!a.bslot || !a.bcount || !a.yp || max_entries == 0 || max_entries > 65535) return hipErrorInvalidValue;
     return a.down_type == T_Q6_K ? go_b_grp_any<Q6K>(a, max_entries, s) : go_b_grp_any<Q4K>(a, max_entries, s);
 }
 

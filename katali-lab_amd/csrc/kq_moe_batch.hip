@@ -44,26 +44,27 @@ constexpr uint32_t MB_MAX_P = MB_MAX_T * MB_MAX_S;
 constexpr uint32_t MB_MAX_E = 513;   // routed experts + the shared expert's virtual id
 
 // meta layout (int32): [0] small entries, [1] grouped-GEMM entries, [2]
-// error bits, [16 ..) small entries (3 ints each: expert, first, count <= 8;
-// at most P), then grouped-GEMM entries (MB_REC ints each: expert, first,
-// count <= 16, 0, then the entry's 16 pairs inline, slots past count
-// holding pair 0; at most P; an expert's entries are consecutive), then
-// order (the P pairs grouped by expert, experts ascending; the order inside
-// one expert's run is arbitrary); a small entry's pairs are
-// order[first .. first + count). A grouped-GEMM tile reads its entry count
-// and its whole record at once: no load waits on another.
+// error bits, [16 ..) small entries (GRP_REC ints each: expert, count <= 8,
+// 0, 0, then the entry's 8 pairs; at most P), then grouped-GEMM entries
+// (MB_REC ints each: expert, 0, count <= 16, 0, then the entry's 16 pairs; at
+// most P; an expert's entries are consecutive). Pair slots past the count
+// hold pair 0; the order of an expert's pairs is arbitrary. A workgroup reads
+// its list's entry count and its whole record at once: no load waits on
+// another.
 constexpr uint32_t MB_GRP = 8;   // pairs per small entry (the grouped GEMV kernels' GRP_MAX)
 constexpr uint32_t MB_BIG = 16;  // pairs per grouped-GEMM entry (the MFMA's 16 B columns)
 constexpr uint32_t MB_FORK_PAIRS = 96;   // batches from this many pairs run the two paths side by side
 constexpr uint32_t MB_DN_CHUNK = 8;   // h blocks staged at once by the down kernel beyond 3 blocks
 constexpr uint32_t MB_REC = 20;      // ints per grouped-GEMM entry: 4 + MB_BIG pairs
 __host__ __device__ inline uint32_t mb_small_off() { return 16; }
-// the grouped-GEMM records start on a 16-byte boundary (each is read as
-// int4s, MB_REC a multiple of 4): the small entries' 3 P ints rounded up
-__host__ __device__ inline uint32_t mb_big_off(uint32_t P) { return 16 + ((3 * P + 3) & ~3u); }
-__host__ __device__ inline uint32_t mb_order_off(uint32_t P) { return mb_big_off(P) + MB_REC * P; }
-static_assert(MB_REC % 4 == 0, "grouped-GEMM records: whole int4s");
-uint64_t moe_batch_meta_words(uint32_t P) { return mb_order_off(P) + P; }
+// (records are whole int4s on 16-byte boundaries)
+__host__ __device__ inline uint32_t mb_big_off(uint32_t P) { return mb_small_off() + GRP_REC * P; }
+static_assert(MB_REC % 4 == 0 && GRP_REC % 4 == 0, "entry records: whole int4s");
+static_assert(GRP_REC == 4 + MB_GRP, "small entries: the pairs inline");
+// Past the small records: entry indices up to the grid's (P / 8 + one per
+// expert, above P only when P is below the expert count) read their record
+// before they know that they have none.
+uint64_t moe_batch_meta_words(uint32_t P) { return mb_big_off(P) + MB_REC * P; }
 
 // Inclusive prefix sum over the 64 lanes of a wave on the VALU: row_shr 1, 2,
 // 4, 8 inside each 16-lane row (lanes without a source add 0), then
@@ -100,9 +101,9 @@ __global__ void __launch_bounds__(1024) k_mb_group(const int32_t *__restrict__ i
         }
         return;
     }
-    __shared__ int32_t cnt[MB_MAX_E], off_all[MB_MAX_E], small_idx[MB_MAX_E], big_idx[MB_MAX_E], cur[MB_MAX_E];
+    __shared__ int32_t cnt[MB_MAX_E], small_idx[MB_MAX_E], big_idx[MB_MAX_E], cur[MB_MAX_E];
     __shared__ int32_t exp_of[MB_MAX_P];
-    __shared__ int32_t wsum[3][16];
+    __shared__ int32_t wsum[2][16];
     __shared__ int32_t bad;
     const uint32_t P = T * S, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const uint32_t NE = n_expert + 1;   // id n_expert = the shared expert
@@ -124,27 +125,23 @@ __global__ void __launch_bounds__(1024) k_mb_group(const int32_t *__restrict__ i
     }
     __syncthreads();
     // Exclusive prefix sums over the experts (NE <= 1024: one per thread) of
-    // the pair counts, the small entry counts and the grouped-GEMM entry
-    // counts.
+    // the small entry counts and the grouped-GEMM entry counts.
     {
         const int c = tid < NE ? cnt[tid] : 0;
         const bool big = c >= (int)min_big && c > 0;
-        const int va = c, vs = big ? 0 : (c + (int)MB_GRP - 1) / (int)MB_GRP, vb = big ? (c + (int)MB_BIG - 1) / (int)MB_BIG : 0;
-        const int ia = wave_incl_scan(va), is = wave_incl_scan(vs), ib = wave_incl_scan(vb);
+        const int vs = big ? 0 : (c + (int)MB_GRP - 1) / (int)MB_GRP, vb = big ? (c + (int)MB_BIG - 1) / (int)MB_BIG : 0;
+        const int is = wave_incl_scan(vs), ib = wave_incl_scan(vb);
         if (lane == 63) {
-            wsum[0][wave] = ia;
-            wsum[1][wave] = is;
-            wsum[2][wave] = ib;
+            wsum[0][wave] = is;
+            wsum[1][wave] = ib;
         }
         __syncthreads();
-        int pa = 0, ps = 0, pb = 0;
+        int ps = 0, pb = 0;
         for (uint32_t w = 0; w < wave; w++) {
-            pa += wsum[0][w];
-            ps += wsum[1][w];
-            pb += wsum[2][w];
+            ps += wsum[0][w];
+            pb += wsum[1][w];
         }
         if (tid < NE) {
-            off_all[tid] = pa + ia - va;
             small_idx[tid] = vs > 0 ? ps + is - vs : -1;   // first small entry of this expert
             big_idx[tid] = big ? pb + ib - vb : -1;   // first entry of this expert
         }
@@ -156,24 +153,25 @@ __global__ void __launch_bounds__(1024) k_mb_group(const int32_t *__restrict__ i
         }
     }
     __syncthreads();
-    int32_t *small = meta + mb_small_off(), *bigl = meta + mb_big_off(P), *order = meta + mb_order_off(P);
+    int32_t *small = meta + mb_small_off(), *bigl = meta + mb_big_off(P);
     for (uint32_t e = tid; e < NE; e += blockDim.x) {
         const int32_t c = cnt[e];
         if (big_idx[e] >= 0) {
             for (int32_t k = 0; (int32_t)MB_BIG * k < c; k++) {
                 int32_t *rec = bigl + MB_REC * (big_idx[e] + k);
                 rec[0] = (int32_t)e;
-                rec[1] = off_all[e] + (int32_t)MB_BIG * k;
+                rec[1] = 0;
                 rec[2] = min((int32_t)MB_BIG, c - (int32_t)MB_BIG * k);
                 rec[3] = 0;
                 for (uint32_t j = 0; j < MB_BIG; j++) rec[4 + j] = 0;   // pair 0: a valid row to address
             }
         } else if (small_idx[e] >= 0) {
             for (int32_t k = 0; (int32_t)MB_GRP * k < c; k++) {
-                const int32_t i = small_idx[e] + k;
-                small[3 * i + 0] = (int32_t)e;
-                small[3 * i + 1] = off_all[e] + (int32_t)MB_GRP * k;
-                small[3 * i + 2] = min((int32_t)MB_GRP, c - (int32_t)MB_GRP * k);
+                int32_t *rec = small + GRP_REC * (small_idx[e] + k);
+                rec[0] = (int32_t)e;
+                rec[1] = min((int32_t)MB_GRP, c - (int32_t)MB_GRP * k);
+                rec[2] = rec[3] = 0;
+                for (uint32_t j = 0; j < MB_GRP; j++) rec[4 + j] = 0;
             }
         }
     }
@@ -184,8 +182,8 @@ __global__ void __launch_bounds__(1024) k_mb_group(const int32_t *__restrict__ i
     for (uint32_t p = tid; p < P; p += blockDim.x) {
         const int32_t e = exp_of[p];
         const int32_t k = atomicAdd(&cur[e], 1);
-        order[off_all[e] + k] = (int32_t)p;
         if (big_idx[e] >= 0) bigl[MB_REC * (big_idx[e] + k / (int32_t)MB_BIG) + 4 + k % (int32_t)MB_BIG] = (int32_t)p;
+        else small[GRP_REC * (small_idx[e] + k / (int32_t)MB_GRP) + 4 + k % (int32_t)MB_GRP] = (int32_t)p;
     }
 }
 
@@ -779,7 +777,6 @@ hipError_t launch_moe_batch(const MoeArgs &base, uint32_t T, uint32_t min_big, c
     a.bS = S;
     a.bslot = meta + mb_small_off();
     a.bcount = meta;
-    a.border = meta + mb_order_off(P);
     // small entries: at most P / 8 + one per expert (each has >= 1 pair)
     const uint32_t ne = base.n_expert + 1;
     const uint32_t max_small = P / MB_GRP + (ne < P ? ne : P);
