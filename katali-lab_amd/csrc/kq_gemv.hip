@@ -319,16 +319,30 @@ constexpr GemvShape gemv_shape(uint32_t items, uint32_t nmax, bool large) {
         }
     return {64, nmax};
 }
+// The shapes of every row length, formed at compile time: a launch of a few
+// microseconds would notice the divisions.
+struct GemvShapes {
+    GemvShape s[GEMV_MAX_COLS / 256 + 1][2];
+};
+template <class QT>
+constexpr GemvShapes gemv_shapes() {
+    GemvShapes t{};
+    for (uint32_t nb = 1; nb <= GEMV_MAX_COLS / 256; nb++)
+        for (int l = 0; l < 2; l++) t.s[nb][l] = gemv_shape(nb * QT::IPB, gemv_nmax<QT>(), l != 0);
+    return t;
+}
+template <class QT>
+inline constexpr GemvShapes GEMV_SHAPES = gemv_shapes<QT>();
 // large: from 6144 items per CU (between 0.8 and 2.4 million measured)
 template <class QT>
 constexpr GemvShape gemv_shape(uint64_t rows, uint64_t cols, uint64_t cus) {
-    const uint32_t items = (uint32_t)(cols / 256) * QT::IPB;
-    return gemv_shape(items, gemv_nmax<QT>(), rows > 6144 * cus / items);
+    const uint64_t nb = cols / 256;
+    return GEMV_SHAPES<QT>.s[nb][rows * nb * QT::IPB > 6144 * cus];
 }
 // the item counts that the two formats have at one and the same row length
 constexpr bool gemv_pair(uint32_t n4, uint32_t n6) {
-    for (uint64_t cols = 256; cols <= GEMV_MAX_COLS; cols += 256)
-        if (gemv_shape<Q4K>(0, cols, 1).N == n4 && gemv_shape<Q6K>(0, cols, 1).N == n6) return true;
+    for (uint64_t nb = 1; nb <= GEMV_MAX_COLS / 256; nb++)
+        if (GEMV_SHAPES<Q4K>.s[nb][0].N == n4 && GEMV_SHAPES<Q6K>.s[nb][0].N == n6) return true;
     return false;
 }
 
@@ -348,6 +362,7 @@ struct GemvGrid {
     uint32_t nw, cap;
 };
 static GemvGrid gemv_grid(uint64_t waves, uint64_t cols, uint32_t cus) {
+    if (waves <= 4ull * cus) return {4, 8};   // no count puts fewer than 4 on a CU
     if (waves > 64ull * cus) return {8, 4};
     if (waves > 16ull * cus) return cols > 2048 ? GemvGrid{8, 2} : GemvGrid{4, 8};
     GemvGrid best{4, 8};
