@@ -189,10 +189,10 @@ constexpr uint32_t FSYNC_XR = FSYNC_XSP + 2 * XCD_MAX_HIDDEN;
 // generations are the XCD layer's.
 constexpr uint32_t FSYNC_XY = FSYNC_XR + FSYNC_REP * 2 * 512;
 constexpr uint32_t FSYNC_XF = FSYNC_XY + 2 * 2 * XCD_MAX_HIDDEN;
-// From FSYNC_DHC, kernel A's half units (a dense FFN): one counter per q8_1
-// block of h (DH_MAX_BLOCKS; every call adds 2 per block), then from
+// From FSYNC_DHC, kernel A's half units: one counter per q8_1 block of h
+// (DH_MAX_BLOCKS; every call adds 2 per block), then from
 // FSYNC_DHW each block's 32 values as words {float, generation}.
-constexpr uint32_t DH_MAX_BLOCKS = 512;   // ffn <= 16384
+constexpr uint32_t DH_MAX_BLOCKS = 1024;   // blocks of all slots
 constexpr uint32_t FSYNC_DHC = FSYNC_XF + 2 * XCD_G;
 constexpr uint32_t FSYNC_DHW = FSYNC_DHC + DH_MAX_BLOCKS;
 constexpr uint32_t fsync_words() { return FSYNC_DHW + 2 * 32 * DH_MAX_BLOCKS; }

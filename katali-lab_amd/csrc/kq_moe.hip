@@ -1047,8 +1047,8 @@ __device__ __forceinline__ void normed_prologue(const MoeArgs &a, uint8_t *area,
 struct NoMore {
     __device__ void operator()(const GuRoute &) const {}
 };
-// HALF (a dense FFN, when 32-row units would leave CUs with uneven counts
-// of workgroups): the workgroup takes half of a unit, 16 gate + 16 up rows,
+// HALF (a dense FFN, or hidden 4096, when 32-row units would leave CUs with
+// uneven counts of workgroups): the workgroup takes half of a unit, 16 gate + 16 up rows,
 // 16 values of the q8_1 block of h. Workgroups b and b + 8 of each run of
 // 16 (one XCD) take the two halves of one block. Each publishes its 16
 // values as tagged words; one atomic per block (a counter that every call
@@ -1061,7 +1061,7 @@ __device__ __forceinline__ void gu_unit(const MoeArgs &a, uint32_t unit, uint8_t
                                         uint32_t *hx = nullptr, After after = After()) {
     // FUSED: flag is this call's generation; h's words are tagged flag + 1
     // and go to hx + 2 * (9 * unit + k), k < 9.
-    static_assert(!(HALF && (FUSED || NORMED)), "half units: the plain dense FFN");
+    static_assert(!(HALF && (FUSED || NORMED)), "half units: plain layers");
     constexpr int RW = HALF ? a1_rw<NB>() / 2 : a1_rw<NB>();
     constexpr int HR = HALF ? 16 : 32;         // gate (and up) rows of the workgroup
     constexpr int NT = a1_threads<NB>();
@@ -3075,7 +3075,7 @@ hipError_t launch_moe_stack(const MoeArgs &a, const StackLayer *lt, uint32_t n_l
 
 uint64_t moe_route_words() { return 2 * MAX_SLOTS; }
 
-// KATALI_HIP_HALF_UNITS=0: kernel A keeps whole units on a dense FFN
+// KATALI_HIP_HALF_UNITS=0: kernel A keeps whole units
 static bool env_half_off() {
     const char *e = getenv("KATALI_HIP_HALF_UNITS");
     return e && (e[0] == '0' || e[0] == 'n' || e[0] == 'N');
@@ -3089,8 +3089,12 @@ static hipError_t go_a(const MoeArgs &a, uint32_t n_slots, hipStream_t s) {
     uint32_t lds = L.total;
     if (NORMED && L.scl + normed_area_bytes(a.hidden) > lds) lds = L.scl + normed_area_bytes(a.hidden);
     if constexpr (!NORMED && NB >= 8) {   // hidden 2048 and 4096
-        if (a.n_sel == 0 && a.fsync && half_units(units, (uint32_t)device_cu_count()) &&
-            units <= DH_MAX_BLOCKS && !env_half_off()) {
+        // Routed layers too at hidden 4096 (8-wave workgroups, two per CU: 288
+        // units 17.4 -> 15.3 us, 896 units 31.3 -> 30.4); at 2048 a half unit
+        // is 16 waves that route for half the rows, and loses (320 units 10.2
+        // -> 14.0 us).
+        if ((a.n_sel == 0 || (NB == 16 && a.n_expert <= 128)) && a.fsync &&
+            half_units(units, (uint32_t)device_cu_count()) && units <= DH_MAX_BLOCKS && !env_half_off()) {
             hipLaunchKernelGGL((k_moe_gu<NB, 2, false, true>), dim3(2 * units), dim3(a1_threads<NB>()),
                                lds_a(a.hidden, NB, 32).total, s, a);
             return hipGetLastError();
