@@ -695,10 +695,22 @@ __global__ void __launch_bounds__(256) k_mb_combine(const float *__restrict__ yp
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= (uint64_t)T * hidden) return;
     const uint32_t t = (uint32_t)(i / hidden), row = (uint32_t)(i % hidden);
+    // eight slots' loads in flight at a time (slots past S load the last one
+    // and are dropped): one by one they were a round trip per slot
+    const float *wt = n_sel ? w + t * n_sel : yp;   // (without routed slots: any valid word, unused)
+    const float *yt = yp + (uint64_t)t * S * hidden + row;
     float acc = 0.0f;
-    for (uint32_t r = 0; r < S; r++) {
-        const float wr = r < n_sel ? w[t * n_sel + r] : 1.0f;
-        acc = fmaf(wr, yp[((uint64_t)t * S + r) * hidden + row], acc);
+    for (uint32_t r0 = 0; r0 < S; r0 += 8) {
+        float v[8], wr[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) {
+            const uint32_t r = min(r0 + k, S - 1);
+            v[k] = yt[(uint64_t)r * hidden];
+            wr[k] = wt[n_sel ? min(r, n_sel - 1) : 0u];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++)
+            if (r0 + k < S) acc = fmaf(r0 + k < n_sel ? wr[k] : 1.0f, v[k], acc);
     }
     y[i] = acc;
 }
