@@ -89,6 +89,8 @@ static hipError_t norm_run(float *x, const float *delta, float scale, const floa
         hipLaunchKernelGGL(kern, dim3(1), dim3(NORM_THREADS), 0, s, x, delta, scale, unit, w, n, eps, out);
         return hipGetLastError();
     };
+    // a weight vector that the residual step updates is read behind the update
+    if (ADD && w < x + n && x < w + n) return go(k_rmsnorm<ADD, 0>);
     if (n <= NORM_THREADS) return go(k_rmsnorm<ADD, 1>);
     if (n <= 2 * NORM_THREADS) return go(k_rmsnorm<ADD, 2>);
     if (n <= 4 * NORM_THREADS) return go(k_rmsnorm<ADD, 4>);
