@@ -363,8 +363,10 @@ int katali_hip_moe_layer_debug(const KataliHipMoe *moe, const KataliHipMoeRoute 
  * an expert with at least mfma_min_tokens pairs runs as an int8 MFMA grouped
  * GEMM, the others through the grouped v_dot4 GEMV kernels (one read of the
  * expert's weights for up to 8 of its tokens); results are identical in
- * definition (q8_1 x and h, rank-order weighted sum), and a one-token batch
- * is bit-identical to katali_hip_moe_layer with the same experts. */
+ * definition (q8_1 x and h, rank-order weighted sum), and a token whose
+ * experts all run through the GEMV kernels (a one-token batch, at the default
+ * threshold) is bit-identical to katali_hip_moe_layer with the same experts on
+ * the two-launch path (the one-launch layers sum down rows over another split). */
 typedef struct KataliHipMoeBatch {
     uint32_t struct_size;                  /* sizeof(KataliHipMoeBatch) */
     uint32_t n_tokens;                     /* T, 1..64 */

@@ -6,11 +6,13 @@
 #include <type_traits>
 
 #include "kq_device.h"
+#include "kq_launch.h"
 
 namespace kq {
 
-// An activation in LDS, laid out for the lanes that read it. A lane item takes NQ groups of 16 values (Q4_K: sub-blocks 2g and 2g+1;
-// Q6_K: quarters t = 0..3 of a half). Tiles of 16 items hold word after word
+// An activation in LDS, laid out for the lanes that read it. A lane item takes
+// NQ groups of 16 values (Q4_K: sub-blocks 2g and 2g+1; Q6_K: quarters t = 0..3
+// of a half). Tiles of 16 items hold word after word
 // of each group side by side for the 16 items, so the lanes of a row read
 // consecutive 16-byte words at offsets the instruction carries; in the
 // activation's own order they are 64 (fp32) or up to 128 (q8_1) bytes apart,
@@ -19,13 +21,14 @@ namespace kq {
 //              right) float [NQ][16]; words 288 bytes apart, so that the eight
 //              lanes storing one 32-value run hit distinct banks
 //   MODE 1, 2  int8 x 16 [NQ][16], the q8_1 blocks' d float [NQ][8], the
-//              groups' exact sums int [NQ][16]
+//              groups' exact sums int [NQ][16]: 352 bytes per 256 values, as
+//              in the activation's own order
 template <class QT, int MODE>
 struct XLds {
     static constexpr uint32_t NQ = 16 / QT::IPB;
     static constexpr uint32_t WORD = MODE == 0 ? 288 : 256;
     static constexpr uint32_t D8 = NQ * WORD, SUM = MODE == 0 ? 4 * NQ * WORD : D8 + NQ * 32;
-    static constexpr uint32_t TILE = (SUM + NQ * 64 + 127) & ~127u;   // whole rows of banks
+    static constexpr uint32_t TILE = SUM + NQ * 64;
     static constexpr uint32_t bytes(uint32_t items) { return (items + 15) / 16 * TILE; }
     // the item and group of 16-value run h (counted along the activation)
     __device__ static __forceinline__ void place(uint32_t h, uint32_t &item, uint32_t &q) {
@@ -115,6 +118,25 @@ __device__ __forceinline__ float item_dot(const Q6K::Raw &r, int c, const XLds<Q
         }
     }
     return acc;
+}
+
+// An entry of the batched layer: up to GRP_MAX (token, rank) pairs of one
+// expert, listed as a record of GRP_REC ints.
+constexpr uint32_t GRP_MAX = 8;
+struct GrpEntry {
+    uint32_t ex, cnt;   // uniform
+    uint32_t pair;      // lane l: pair l % GRP_MAX (pair 0 past the count)
+};
+// The record of entry ei; cnt 0 when the list has no such entry (the record is
+// inside the list's memory all the same).
+__device__ __forceinline__ GrpEntry grp_entry(const MoeArgs &a, uint32_t ei) {
+    const int32_t *rec = a.bslot + (uint64_t)GRP_REC * ei;
+    const int32_t n = *a.bcount, ex = rec[0], cnt = rec[1];
+    GrpEntry e;
+    e.pair = (uint32_t)rec[4 + (threadIdx.x & (GRP_MAX - 1))];
+    e.ex = (uint32_t)__builtin_amdgcn_readfirstlane(ex);
+    e.cnt = ei < (uint32_t)__builtin_amdgcn_readfirstlane(n) ? (uint32_t)__builtin_amdgcn_readfirstlane(cnt) : 0u;
+    return e;
 }
 
 inline int ilog2(uint32_t v) {

@@ -128,9 +128,10 @@ struct MoeArgs {
     uint32_t hloc;
 };
 // Kernel B for rows of more than four blocks (kq_moe_down.hip), after kernel A
-// has written h and the routing; hipErrorNotSupported when the shape is
-// kernel B's own (shorter rows, or h past the LDS in its layout).
+// has written h and the routing.
 hipError_t launch_moe_down_wide(const MoeArgs &a, uint32_t n_slots, hipStream_t s);
+// launch_moe_groups_down for Q4_K rows of more than 16 blocks (kq_moe_down.hip)
+hipError_t launch_moe_groups_down_long(const MoeArgs &a, uint32_t max_entries, hipStream_t s);
 bool moe_shape_supported(uint32_t gate_type, uint32_t down_type, uint32_t hidden, uint32_t ffn);
 // Dynamic LDS (bytes) of the largest workgroup a layer of this shape launches:
 // kernel A, kernel B (n_slots * (ffn + ffn/8 + ffn/4) for the staged h, plus
@@ -140,8 +141,6 @@ bool moe_shape_supported(uint32_t gate_type, uint32_t down_type, uint32_t hidden
 uint32_t moe_layer_lds(uint32_t hidden, uint32_t ffn, uint32_t n_slots);
 uint32_t moe_groups_lds(uint32_t hidden, uint32_t ffn);
 uint32_t moe_batch_lds(uint32_t hidden, uint32_t ffn);
-// gfx950's LDS per workgroup
-constexpr uint32_t LDS_PER_WG = 160 * 1024;
 // The layer in one launch when the shape fits the fused kernel and a.fsync is
 // set (and `allow_fused`), else kernels A and B. *fused tells which ran.
 // allow_xcd: the XCD-sliced one-launch layer where the shape fits it

@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "kq_device.h"
+#include "kq_items.h"
 #include "kq_launch.h"
 
 namespace kq {
@@ -1432,12 +1433,10 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
     const bool routed = (int)sl < a.n_sel;
     const uint8_t *db = routed ? a.down + (uint64_t)sid * a.hidden * rbd : a.down_sh;
     const uint8_t *rp = db + (uint64_t)(row0 + r) * rbd;
-    typename QD::RawQ raw[IPL > 0 ? IPL : 1];   // (the lanes of a quad hold one block's items)
-    if constexpr (IPL > 0) {
+    typename QD::RawQ raw[IPL];   // (the lanes of a quad hold one block's items)
 #pragma unroll
-        for (int i = 0; i < IPL; i++)   // clamped: a block past the row is loaded and dropped
-            raw[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
-    }
+    for (int i = 0; i < IPL; i++)   // clamped: a block past the row is loaded and dropped
+        raw[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
     stage_h(lds + L.hacts, a.ffn, ntask, 0, nt, hv);
     for (uint32_t first = HT * nt; first < ntask; first += HT * nt) {
         load_h(a.hq8, ntask, first, nt, hv);   // only when n_slots * ffn / 16 > nt * HT
@@ -1447,15 +1446,11 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
     float x = 0.0f;
     {
         const Act act = act_carve(lds + L.hacts + sl * act_bytes(a.ffn), a.ffn);
-        if constexpr (IPL > 0) {
 #pragma unroll
-            for (int i = 0; i < IPL; i++) {
-                const uint32_t b = sub + P * i;
-                const float v = QD::dot_q8(QD::full(raw[i]), (int)item, act, min(b, nbk - 1));
-                x += b < nbk ? v : 0.0f;
-            }
-        } else {
-            for (uint32_t b = sub; b < nbk; b += P) x += QD::dot_q8(QD::load(rp + b * QD::BB, (int)item), (int)item, act, b);
+        for (int i = 0; i < IPL; i++) {
+            const uint32_t b = sub + P * i;
+            const float v = QD::dot_q8(QD::full(raw[i]), (int)item, act, min(b, nbk - 1));
+            x += b < nbk ? v : 0.0f;
         }
     }
     x = group_sum<S>(x);
@@ -1494,24 +1489,6 @@ __global__ void __launch_bounds__(NT > 0 ? NT : B_MAX_THREADS) k_moe_down(MoeArg
 // activations issued behind the weights, after a load of their pairs, came two
 // round trips after the last weight.
 // ---------------------------------------------------------------------------
-constexpr uint32_t GRP_MAX = 8;
-
-struct GrpEntry {
-    uint32_t ex, cnt;   // uniform
-    uint32_t pair;      // lane l: pair l % GRP_MAX (pair 0 past the count)
-};
-// The record of entry ei; cnt 0 when the list has no such entry (the record is
-// inside the list's memory all the same).
-__device__ __forceinline__ GrpEntry grp_entry(const MoeArgs &a, uint32_t ei) {
-    const int32_t *rec = a.bslot + (uint64_t)GRP_REC * ei;
-    const int32_t n = *a.bcount, ex = rec[0], cnt = rec[1];
-    GrpEntry e;
-    e.pair = (uint32_t)rec[4 + (threadIdx.x & (GRP_MAX - 1))];
-    e.ex = (uint32_t)__builtin_amdgcn_readfirstlane(ex);
-    e.cnt = ei < (uint32_t)__builtin_amdgcn_readfirstlane(n) ? (uint32_t)__builtin_amdgcn_readfirstlane(cnt) : 0u;
-    return e;
-}
-
 // One 16-byte half block of a pair's q8_1 row: half block r of pair g
 struct GrpX {
     uint4 q;
@@ -1700,7 +1677,8 @@ __global__ void __launch_bounds__(A_THREADS) k_moe_gu_grp(MoeArgs a) {
 
 // Down for an entry: kernel B's tile (tr rows, S = IPB * P lanes per row, the
 // same blocks per lane), every pair's h staged in LDS, each pair's unweighted
-// output row to yp.
+// output row to yp. Q4_K rows above 16 blocks have their own kernel
+// (k_moe_down_grp_long).
 template <class QD, int IPL, int P>
 __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
     extern __shared__ __align__(16) uint8_t lds[];
@@ -1741,11 +1719,9 @@ __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
     const uint32_t r = min(ls, nrows - 1);   // idle lane-slots load a real row and drop it
     const uint8_t *db = ex >= a.n_expert ? a.down_sh : a.down + (uint64_t)ex * a.hidden * rbd;
     const uint8_t *rp = db + (uint64_t)(row0 + r) * rbd;
-    typename QD::RawQ rawq[IPL > 0 ? IPL : 1];   // (the lanes of a quad hold one block's items)
-    if constexpr (IPL > 0) {
+    typename QD::RawQ rawq[IPL];   // (the lanes of a quad hold one block's items)
 #pragma unroll
-        for (int i = 0; i < IPL; i++) rawq[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
-    }
+    for (int i = 0; i < IPL; i++) rawq[i] = QD::load_quad(rp + min(sub + P * i, nbk - 1) * QD::BB, (int)item);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);   // every weight load is out before h is staged
     auto h_put = [&](uint32_t t, const GrpX &v) {
@@ -1761,29 +1737,23 @@ __global__ void __launch_bounds__(256) k_moe_down_grp(MoeArgs a, uint32_t tr) {
         if (tid + t0 < ntask) h_put(tid + t0, v);
     }
     // the quants are unpacked once for all pairs
-    typename QD::Raw raw[IPL > 0 ? IPL : 1];
-    typename QD::Unp unp[IPL > 0 ? IPL : 1];
-    if constexpr (IPL > 0) {
+    typename QD::Raw raw[IPL];
+    typename QD::Unp unp[IPL];
 #pragma unroll
-        for (int i = 0; i < IPL; i++) {
-            raw[i] = QD::full(rawq[i]);
-            unp[i] = QD::unpack(raw[i]);
-        }
+    for (int i = 0; i < IPL; i++) {
+        raw[i] = QD::full(rawq[i]);
+        unp[i] = QD::unpack(raw[i]);
     }
     __syncthreads();
     const uint32_t ab = act_bytes(a.ffn);
     for (uint32_t g = 0; g < cnt; g++) {
         const Act act = act_carve(lds + g * ab, a.ffn);
         float x = 0.0f;
-        if constexpr (IPL > 0) {
 #pragma unroll
-            for (int i = 0; i < IPL; i++) {
-                const uint32_t b = sub + P * i;
-                const float v = QD::dot_q8_u(raw[i], unp[i], (int)item, act, min(b, nbk - 1));
-                x += b < nbk ? v : 0.0f;
-            }
-        } else {
-            for (uint32_t b = sub; b < nbk; b += P) x += QD::dot_q8(QD::load(rp + b * QD::BB, (int)item), (int)item, act, b);
+        for (int i = 0; i < IPL; i++) {
+            const uint32_t b = sub + P * i;
+            const float v = QD::dot_q8_u(raw[i], unp[i], (int)item, act, min(b, nbk - 1));
+            x += b < nbk ? v : 0.0f;
         }
         x = group_sum<S>(x);
         const uint32_t pair = (uint32_t)__builtin_amdgcn_readlane((int)ent.pair, (int)g);
@@ -3139,8 +3109,7 @@ static hipError_t go_b(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, hipS
 }
 // P = lanes-per-pair multiplier: the smallest power of two that brings a
 // lane's blocks (IPL = ceil(nb / P)) to at most 4 while a workgroup still
-// holds every slot of at least one output row; 1 (a runtime block loop when
-// IPL > 4) where no unrolled variant fits.
+// holds every slot of at least one output row; 1 where no variant fits.
 template <class QD>
 static uint32_t b_mult(uint32_t nb, uint32_t n_slots) {
     uint32_t p = 1;
@@ -3151,7 +3120,7 @@ static uint32_t b_mult(uint32_t nb, uint32_t n_slots) {
 }
 // The switch key of kernel B's unrolled variants, P * 8 + IPL, unique only
 // for IPL <= 4 (P = 1 with 26 blocks would otherwise read as P = 4, IPL = 2);
-// 0 (the runtime block loop) for every other choice.
+// 0 (the kernels for long rows, kq_moe_down.hip) for every other choice.
 static uint32_t b_variant(uint32_t p, uint32_t ipl) { return ipl >= 1 && ipl <= 4 ? p * 8 + ipl : 0; }
 
 // Kernel B's variant and tiles: 256-thread tiles, unless those give between
@@ -3203,18 +3172,16 @@ static hipError_t go_b_any(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, 
             default: break;
         }
     }
-    return go_b<QD, 0, 1>(a, n_slots, pl, s);
+    return hipErrorInvalidValue;
 }
 static hipError_t go_b_run(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, hipStream_t s) {
-    // What would run the runtime block loop, and the whole-wave rows of two
-    // and more slots, have their own kernel (two slots of 14336, Q6_K: 25.8 ->
-    // 22.2 us; six of 9728, Q4_K: 39.8 -> 18.0; ten of 4096, Q4_K: 38.1 ->
-    // 14.2). One slot (a dense FFN) has one pair per wave there and gains
-    // nothing: 10.9 us here at 12288, 11.4 there.
-    if (pl.key == 0 || (pl.key >= 16 * 8 && n_slots > 1)) {
-        const hipError_t e = launch_moe_down_wide(a, n_slots, s);
-        if (e != hipErrorNotSupported) return e;
-    }
+    // What no unrolled variant takes, and the whole-wave rows of two and more
+    // slots, have their own kernel (two slots of 14336, Q6_K: 25.8 -> 22.2 us;
+    // six of 9728, Q4_K: 39.8 -> 18.0; ten of 4096, Q4_K: 38.1 -> 14.2). One
+    // slot (a dense FFN) has one pair per wave there and gains nothing: 10.9
+    // us here at 12288, 11.4 there. Both give a pair the same lane split, the
+    // grouped kernels' too, so its sum has the same bits in all of them.
+    if (pl.key == 0 || (pl.key >= 16 * 8 && n_slots > 1)) return launch_moe_down_wide(a, n_slots, s);
     return a.down_type == T_Q6_K ? go_b_any<Q6K>(a, n_slots, pl, s) : go_b_any<Q4K>(a, n_slots, pl, s);
 }
 
@@ -3434,7 +3401,8 @@ static hipError_t go_b_grp_any(const MoeArgs &a, uint32_t max_entries, hipStream
             default: break;
         }
     }
-    return go_b_grp<QD, 0, 1>(a, max_entries, s);
+    if constexpr (QD::TYPE == T_Q4_K) return launch_moe_groups_down_long(a, max_entries, s);
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_moe_groups_down(const MoeArgs &a, uint32_t max_entries, hipStream_t s) {

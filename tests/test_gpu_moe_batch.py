@@ -133,6 +133,43 @@ def test_moe_batch_single_token_matches_layer(hip, oracle, built):
     assert np.array_equal(y1.download(np.uint32), y2.download(np.uint32))
 
 
+# ffn, slots (the last one shared), down_type: rows above 16 blocks, whose
+# down kernels the two paths choose on their own
+LONG = [(f, k, False, t) for t, fs in ((Q4_K, (4352, 6912, 14336)), (Q6_K, (4352, 14336))) for f in fs for k in (1, 2, 6)] + [
+    (4352, 9, False, Q4_K), (4352, 16, True, Q4_K), (6912, 16, True, Q4_K), (14336, 8, False, Q4_K),   # h near the LDS limit
+    (4352, 16, True, Q6_K), (6912, 16, True, Q6_K), (14592, 7, True, Q6_K),
+    (4096, 9, False, Q4_K), (2304, 12, False, Q4_K), (1536, 16, True, Q6_K)]   # up to 16 blocks, many slots
+
+
+@pytest.mark.parametrize("ffn,n_sel,shared,down_type", LONG,
+                         ids=[f"f{c[0]}_k{c[1]}{'_sh' if c[2] else ''}{'_q4' if c[3] == Q4_K else '_q6'}" for c in LONG])
+def test_moe_batch_single_token_matches_layer_long_rows(hip, ffn, n_sel, shared, down_type):
+    """The same for long down rows: a pair's lane split is one for both paths
+    (so the tokens of a larger batch on the GEMV kernels have those bits too)."""
+    print(f"[moe-batch] long rows, ffn={ffn} k={n_sel} shared={shared} down={down_type}", flush=True)
+    hidden, n_exp = 256, n_sel + 1
+
+    def mat(n, t, r, c):
+        b = hip.alloc(n * r * (c // 256) * (144 if t == Q4_K else 210))
+        hip.synth_fill(t, b, n * r * (c // 256), n + r + c + t)
+        return b
+    dev = [mat(n_exp, t, r, c) for t, r, c in ((Q4_K, ffn, hidden), (Q4_K, ffn, hidden), (down_type, hidden, ffn))]
+    sh = [mat(1, t, r, c) for t, r, c in ((Q4_K, ffn, hidden), (Q4_K, ffn, hidden), (down_type, hidden, ffn))] if shared else None
+    desc = hip.moe_desc(hidden, ffn, n_exp, *dev, down_type=down_type, shared=sh)
+    rng = np.random.default_rng(ffn + n_sel)
+    for T in (1, 11):   # 11: experts of more than one pair, and of more than one entry of 8
+        ids, w = zipf_routes(rng, T, n_exp, n_sel)
+        x = rng.standard_normal((T, hidden)).astype(np.float32)
+        yb, y1 = hip.alloc(T * hidden * 4), hip.alloc(hidden * 4)
+        hip.moe_batch(desc, T, n_sel, hip.to_device(ids), hip.to_device(w), hip.to_device(x), yb, mfma_min_tokens=1000)
+        got = yb.download(np.uint32).reshape(T, hidden)
+        for t in range(T):
+            route = hip.moe_route(n_sel, ids=hip.to_device(ids[t]), weights=hip.to_device(w[t]))
+            hip.moe_layer(desc, route, y1, x=hip.to_device(x[t]))
+            hip.sync()
+            assert np.array_equal(got[t], y1.download(np.uint32)), t
+
+
 def test_moe_batch_rejects_bad_arguments(hip, built):
     from katali_hip import HipError
     case = CASES[4]
