@@ -197,11 +197,15 @@ typedef struct KataliHipMoeRoute {
  * after about 2^20 polls (about a second, per wait, so a call can stall for
  * seconds), reported as KATALI_HIP_E_TIMEOUT by the next katali_hip_sync,
  * the outputs then invalid; from that report on, the library runs every
- * layer on the two-launch path (graphs captured before keep their kernels;
- * katali_hip_one_launch(1) allows the one-launch form again).
- * KATALI_HIP_XCD=0 in the environment keeps such layers on the two-launch
- * path, which never waits in-kernel (KATALI_HIP_XCD_SHARED=0 only the
- * shared-expert shapes). */
+ * layer on the two-launch path without in-kernel waits (graphs captured before
+ * keep their kernels; katali_hip_one_launch(1) allows the waiting forms again).
+ * The two-launch path waits in one case: where the first kernel's 32-row units
+ * would leave the CUs uneven counts (a dense FFN of hidden 2048 or 4096, any
+ * layer of hidden 4096 with up to 128 experts) two workgroups share a unit and
+ * the second waits for the values of the first, which is already running.
+ * KATALI_HIP_XCD=0 in the environment keeps every layer on the two-launch
+ * path without such waits (KATALI_HIP_XCD_SHARED=0 only the shared-expert
+ * shapes on the two-launch path). */
 int katali_hip_moe_layer(const KataliHipMoe *moe, const KataliHipMoeRoute *route,
                          const float *x_dev, const void *xq8_dev, float *y_dev);
 
@@ -220,8 +224,9 @@ int katali_hip_moe_layer(const KataliHipMoe *moe, const KataliHipMoeRoute *route
  * wait can expire, reported as KATALI_HIP_E_TIMEOUT by the next
  * katali_hip_sync, the outputs then invalid). When kernel A has more
  * workgroups (n_slots * ffn / 32) than the device has CUs, or n_expert is
- * more than 4 router rows per workgroup, the call runs the norm/router
- * launch and the layer instead, with the same results. Rules of
+ * more than 4 router rows per workgroup, or after an expired wait, the call
+ * runs the norm/router launch and the layer instead, with the same results.
+ * Rules of
  * katali_hip_rmsnorm_matvec_f32
  * (16-byte alignment, outputs apart from inputs) and of katali_hip_moe_layer;
  * n_sel >= 1; xn_out and logits_out may be NULL. No counterpart in the
@@ -299,7 +304,8 @@ int katali_hip_moe_stack_run(void *stack, const float *x_dev, const float *delta
 int katali_hip_moe_stack_destroy(void *stack);
 
 /* The one-launch layers (the XCD-sliced layer, its normed form and the
- * stack), whose workgroups wait for each other: mode 0 turns them off (every
+ * stack), whose workgroups wait for each other, and the waits in kernel A
+ * (shared units, the normed form's exchange): mode 0 turns them off (every
  * layer then runs as kernels A and B, as after an expired wait), 1 turns
  * them back on (after an expiry, once the device is no longer shared), -1
  * only asks. Returns the state before the call: 1 on, 0 off. The

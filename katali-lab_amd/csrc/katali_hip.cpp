@@ -311,9 +311,12 @@ int moe_impl(const KataliHipMoe *m, const KataliHipMoeRoute *r, const float *x, 
     // the XCD-sliced layer is set off before the launch, so its words carry a
     // tag no other workgroup waits for and every wait of that call runs to
     // its bound and expires (about a second); the sync then reports the
-    // expiry and clears the exchange area. Not for capture.
+    // expiry and clears the exchange area. The first block's counter of the
+    // half units too: odd, so its first workgroup waits for the second. Not
+    // for capture.
     if (env_on("KATALI_HIP_TEST_SKEW") && !g_capturing) {
-        const hipError_t e = hipMemsetAsync(g_fsync + kq::FSYNC_X, 0xA5, 4, g_stream);
+        hipError_t e = hipMemsetAsync(g_fsync + kq::FSYNC_X, 0xA5, 4, g_stream);
+        if (e == hipSuccess) e = hipMemsetAsync(g_fsync + kq::FSYNC_DHC, 0xA5, 4, g_stream);
         if (e != hipSuccess) return hip_fail(e, "test skew");
     }
     // Eight slots take the XCD-sliced layer (one launch, every CU streaming
@@ -329,7 +332,8 @@ int moe_impl(const KataliHipMoe *m, const KataliHipMoeRoute *r, const float *x, 
     const bool allow_fused = env_on("KATALI_HIP_FUSED");
     const bool allow_xcd = !env_off("KATALI_HIP_XCD");
     const bool xcd_units = !env_off("KATALI_HIP_XCD_SHARED");
-    rc = launched(kq::launch_moe(a, g_stream, allow_fused, nullptr, allow_xcd, xcd_units), "moe launch");
+    // (KATALI_HIP_XCD=0: no form that waits in-kernel, half units included)
+    rc = launched(kq::launch_moe(a, g_stream, allow_fused, nullptr, allow_xcd, xcd_units, allow_xcd), "moe launch");
     if (rc) return rc;
     if (hq8_dbg) {
         hipError_t e = hipMemcpyAsync(hq8_dbg, g_hq8, hq8_bytes, hipMemcpyDeviceToDevice, g_stream);
@@ -515,16 +519,17 @@ int katali_hip_sync(void) {
     if (na) (void)hipMemset(g_scratch + NOALLOC_ERR, 0, 4);
     if (err) (void)hipMemset(g_err_dev, 0, 4);
     if ((err | na) & 12) {
-        // a one-launch layer gave up waiting for its own workgroups (the
-        // device was shared with other work; bit 4), or one of its
+        // a layer gave up waiting for its own workgroups (the device was
+        // shared with other work; bit 4), or one of a one-launch layer's
         // workgroups ran on another XCD than the round-robin dispatch puts it
         // on (bit 8, whose slot's waits may have expired too): its outputs
         // and the exchange words are void; start over, and from now on run
-        // every layer as kernels A and B, which never wait in-kernel
+        // every layer as kernels A and B in whole units, which never wait
+        // in-kernel
         if (g_fsync && (err & 12)) (void)hipMemset(g_fsync, 0, kq::fsync_words() * 4);
         if (na & 12) (void)hipMemset(g_scratch + NOALLOC_FSYNC, 0, kq::fsync_words() * 4);
         kq::xcd_disable();
-        return fail(KATALI_HIP_E_TIMEOUT, "MoE layer: %s (outputs invalid; the one-launch layers are off from now on)",
+        return fail(KATALI_HIP_E_TIMEOUT, "MoE layer: %s (outputs invalid; the forms that wait in-kernel are off from now on)",
                     ((err | na) & 8) ? "a workgroup ran on another XCD than its slot's" : "in-kernel wait expired");
     }
     if (err | na)
@@ -712,8 +717,9 @@ int katali_hip_moe_layer_noalloc(const KataliHipMoe *m, const KataliHipMoeRoute 
     a.err = (int32_t *)(g_scratch + NOALLOC_ERR);
     a.fsync = (uint32_t *)(g_scratch + NOALLOC_FSYNC);
     // the layer choice of katali_hip_moe_layer (moe_impl), so the outputs are its bits
-    return launched(kq::launch_moe(a, g_stream, env_on("KATALI_HIP_FUSED"), nullptr, !env_off("KATALI_HIP_XCD"),
-                                   !env_off("KATALI_HIP_XCD_SHARED")),
+    const bool allow_xcd = !env_off("KATALI_HIP_XCD");
+    return launched(kq::launch_moe(a, g_stream, env_on("KATALI_HIP_FUSED"), nullptr, allow_xcd,
+                                   !env_off("KATALI_HIP_XCD_SHARED"), allow_xcd),
                     "moe launch");
 }
 

@@ -147,8 +147,11 @@ uint32_t moe_batch_lds(uint32_t hidden, uint32_t ffn);
 // (eight slots, or with xcd_shared_units eight routed experts and the
 // shared expert with ffn 256 or 512; hidden 1024 or 2048, ffn <= 1024,
 // <= 256 experts, a 256-CU device), tried before the fused one.
+// may_wait: kernel A may run half units, whose second workgroup waits for the
+// first's values (never once xcd_disabled()); else kernels A and B wait for
+// nothing.
 hipError_t launch_moe(const MoeArgs &a, hipStream_t s, bool allow_fused = false, bool *fused = nullptr,
-                      bool allow_xcd = false, bool xcd_shared_units = false);
+                      bool allow_xcd = false, bool xcd_shared_units = false, bool may_wait = false);
 // The in-kernel exchanges (zeroed once, before first use): [0] the fused
 // layer's generation, [1] the normed layer's; from FSYNC_H one block per
 // workgroup of the fused layer of 9 8-byte words {dword, generation} (its
@@ -202,10 +205,11 @@ static_assert(FSYNC_H + 2 * 9 * FUSED_MAX_G <= FSYNC_R, "exchange areas overlap"
 // launch_norm_router), exchanges the logits between its workgroups through
 // a.fsync, routes and runs the gate/up units; kernel B as launch_moe's.
 // When the router rows do not spread over kernel A's workgroups (more than
-// 4 rows each), launch_norm_router into xn_buf / logits_buf first, then
-// launch_moe. *merged tells which ran.
+// 4 rows each), or once xcd_disabled(), launch_norm_router into xn_buf /
+// logits_buf first, then launch_moe. *merged tells which ran.
 // allow_xcd: eight-slot layers of the XCD-sliced layer's shapes run as that
-// layer with the steps before it in its prologue, in one launch.
+// layer with the steps before it in its prologue, in one launch; also
+// launch_moe's may_wait.
 hipError_t launch_moe_normed(MoeArgs a, float *xn_buf, float *logits_buf, hipStream_t s, bool *merged = nullptr,
                              bool allow_xcd = false);
 // One layer of the stacked layer (launch_moe_stack): weights, routing and
@@ -240,9 +244,10 @@ struct StackLayer {
 // launch_moe_normed layer by layer. hipErrorNotSupported for shapes the XCD
 // layer does not take (then nothing is launched).
 hipError_t launch_moe_stack(const MoeArgs &a, const StackLayer *lt, uint32_t n_layers, bool normed, hipStream_t s);
-// After an expired in-kernel wait the library stops choosing the layers
-// whose workgroups wait for each other (the XCD-sliced layer and the stack);
-// kernels A and B run every later layer.
+// After an expired in-kernel wait the library stops choosing the forms whose
+// workgroups wait for each other (the XCD-sliced layer and the stack, the
+// normed kernel A, half units); kernels A and B run every later layer, in
+// whole units.
 void xcd_disable();
 void xcd_enable();
 bool xcd_disabled();

@@ -3051,8 +3051,10 @@ static bool env_half_off() {
     return e && (e[0] == '0' || e[0] == 'n' || e[0] == 'N');
 }
 
+// may_wait: half units allowed (the second workgroup of a block polls for the
+// first one's words, which that one writes once it has counted itself in)
 template <int NB, bool NORMED = false>
-static hipError_t go_a(const MoeArgs &a, uint32_t n_slots, hipStream_t s) {
+static hipError_t go_a(const MoeArgs &a, uint32_t n_slots, hipStream_t s, bool may_wait = false) {
     const LdsA L = lds_a(a.hidden, NB);
     const uint32_t units = n_slots * (a.ffn / 32);
     const dim3 grid(units);
@@ -3063,7 +3065,7 @@ static hipError_t go_a(const MoeArgs &a, uint32_t n_slots, hipStream_t s) {
         // units 17.4 -> 15.3 us, 896 units 31.3 -> 30.4); at 2048 a half unit
         // is 16 waves that route for half the rows, and loses (320 units 10.2
         // -> 14.0 us).
-        if ((a.n_sel == 0 || (NB == 16 && a.n_expert <= 128)) && a.fsync &&
+        if (may_wait && !xcd_disabled() && (a.n_sel == 0 || (NB == 16 && a.n_expert <= 128)) && a.fsync &&
             half_units(units, (uint32_t)device_cu_count()) && units <= DH_MAX_BLOCKS && !env_half_off()) {
             hipLaunchKernelGGL((k_moe_gu<NB, 2, false, true>), dim3(2 * units), dim3(a1_threads<NB>()),
                                lds_a(a.hidden, NB, 32).total, s, a);
@@ -3206,7 +3208,7 @@ bool moe_shape_supported(uint32_t gate_type, uint32_t down_type, uint32_t hidden
     return ffn % 256 == 0 && ffn >= 256;
 }
 
-static hipError_t go_a_any(const MoeArgs &a, uint32_t n_slots, hipStream_t s);
+static hipError_t go_a_any(const MoeArgs &a, uint32_t n_slots, hipStream_t s, bool may_wait);
 
 // Routing of T tokens at once (batched prefill): one wave per token runs
 // kernel A's own routing (load_keys, wave_topk, route_weight) on its row of
@@ -3242,7 +3244,7 @@ hipError_t launch_route_batch(const float *logits, uint32_t n_tokens, uint32_t n
 }
 
 hipError_t launch_moe(const MoeArgs &a, hipStream_t s, bool allow_fused, bool *fused, bool allow_xcd,
-                      bool xcd_shared_units) {
+                      bool xcd_shared_units, bool may_wait) {
     if (a.n_expert > MAX_EXPERT || a.n_sel > MAX_SEL) return hipErrorInvalidValue;
     const uint32_t n_slots = (uint32_t)a.n_sel + (a.has_shared ? 1u : 0u);
     if (fused) *fused = false;
@@ -3260,18 +3262,18 @@ hipError_t launch_moe(const MoeArgs &a, hipStream_t s, bool allow_fused, bool *f
             return f;
         }
     }
-    const hipError_t e = go_a_any(a, n_slots, s);
+    const hipError_t e = go_a_any(a, n_slots, s, may_wait);
     if (e != hipSuccess) return e;
     return go_b_run(a, n_slots, b_plan_any(a, n_slots), s);
 }
 
-static hipError_t go_a_any(const MoeArgs &a, uint32_t n_slots, hipStream_t s) {
+static hipError_t go_a_any(const MoeArgs &a, uint32_t n_slots, hipStream_t s, bool may_wait) {
     switch (a.hidden / 256) {
-        case 1: return go_a<1>(a, n_slots, s);
-        case 2: return go_a<2>(a, n_slots, s);
-        case 4: return go_a<4>(a, n_slots, s);
-        case 8: return go_a<8>(a, n_slots, s);
-        case 16: return go_a<16>(a, n_slots, s);
+        case 1: return go_a<1>(a, n_slots, s, may_wait);
+        case 2: return go_a<2>(a, n_slots, s, may_wait);
+        case 4: return go_a<4>(a, n_slots, s, may_wait);
+        case 8: return go_a<8>(a, n_slots, s, may_wait);
+        case 16: return go_a<16>(a, n_slots, s, may_wait);
         default: return hipErrorInvalidValue;
     }
 }
@@ -3303,7 +3305,7 @@ hipError_t launch_moe_normed(MoeArgs a, float *xn_buf, float *logits_buf, hipStr
     const uint32_t U = n_slots * (a.ffn / 32);
     // kernel A's workgroups wait for each other's router rows: all of them
     // must be resident at once (one per CU at most), each with <= 4 rows
-    if (a.fsync && U <= (uint32_t)device_cu_count() && (a.n_expert + U - 1) / U <= NORMED_MAX_R) {
+    if (a.fsync && !xcd_disabled() && U <= (uint32_t)device_cu_count() && (a.n_expert + U - 1) / U <= NORMED_MAX_R) {
         a.x = nullptr;
         a.xq = nullptr;
         a.logits = nullptr;
@@ -3335,7 +3337,7 @@ hipError_t launch_moe_normed(MoeArgs a, float *xn_buf, float *logits_buf, hipStr
     b.xq = nullptr;
     b.logits = lg;
     b.step = nullptr;
-    return launch_moe(b, s);
+    return launch_moe(b, s, false, nullptr, false, false, allow_xcd);
 }
 
 template <int NB>

@@ -61,3 +61,52 @@ def test_half_units_routed(hip, oracle, monkeypatch, ffn, n_exp, k, shared):
             assert np.array_equal(y.download(np.uint32), out["half", "logits"][0]), rep
     finally:
         hip.graph_destroy(gr)
+
+
+@pytest.mark.parametrize("ffn,n_exp,k,shared", [CASES[0], (12288, 1, 0, True)])
+def test_half_units_off_where_nothing_waits(hip, monkeypatch, ffn, n_exp, k, shared):
+    """KATALI_HIP_TEST_SKEW=1 sets block 0's counter odd, so its first
+    workgroup waits for the second and that wait runs to its bound (about a
+    second) and expires. KATALI_HIP_XCD=0, a reported expiry and
+    katali_hip_one_launch(0) promise kernels that wait for nothing: there the
+    skew changes nothing."""
+    import katali_hip as K
+    print(f"[moe_half_waits] ffn={ffn} k={k} shared={shared}", flush=True)
+    hidden = 4096
+
+    def mats(n):
+        bufs = []
+        for t, r, c in ((Q4_K, ffn, hidden), (Q4_K, ffn, hidden), (Q6_K, hidden, ffn)):
+            nb = n * r * (c // 256)
+            bufs.append(hip.alloc(nb * K.BLOCK_BYTES[t]))
+            hip.synth_fill(t, bufs[-1], nb, n + r + t)
+        return bufs
+    desc = hip.moe_desc(hidden, ffn, n_exp, *mats(n_exp), down_type=Q6_K, shared=mats(1) if shared else None)
+    rng = np.random.default_rng(ffn)
+    x = hip.to_device(S.activation(rng, hidden))
+    dl = hip.to_device(rng.standard_normal(n_exp).astype(np.float32))
+    route, y = hip.moe_route(k, logits=dl) if k else hip.moe_route(0), hip.alloc(hidden * 4)
+
+    def run():
+        hip.moe_layer(desc, route, y, x=x)
+        hip.sync()
+        return y.download(np.uint32)
+    ref = run()
+    monkeypatch.setenv("KATALI_HIP_TEST_SKEW", "1")
+    try:
+        monkeypatch.setenv("KATALI_HIP_XCD", "0")
+        assert np.array_equal(run(), ref)
+        monkeypatch.delenv("KATALI_HIP_XCD")
+        hip.one_launch(0)
+        assert np.array_equal(run(), ref)
+        hip.one_launch(1)
+        with pytest.raises(K.HipError) as err:   # the hook does reach half units
+            run()
+        assert err.value.rc == K.E_TIMEOUT, err.value
+        monkeypatch.delenv("KATALI_HIP_TEST_SKEW")
+        assert not hip.one_launch(-1)
+        assert np.array_equal(run(), ref)
+    finally:
+        hip.one_launch(1)
+    for _ in range(3):
+        assert np.array_equal(run(), ref)
