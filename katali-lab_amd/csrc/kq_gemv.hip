@@ -13,8 +13,9 @@
 // by its converts and FMAs, about 110 per 18 bytes: 40000 x 5120 4.0 TB/s), by
 // launch, first loads and tail below about 20 MB. Row lengths that are no
 // power of two used to run a loop over items with one load in flight and as
-// few as 4 lanes per row (Q6_K 5120 x 13824, fp32: 50.4 us, now 19.9; Q4_K
-// 9731 x 2560: 8.9, now 5.6; q, k, v of 2560 columns: 10.1, now 6.5).
+// few as 4 lanes per row (weights from memory: Q6_K 5120 x 13824, fp32, 50.4 us,
+// now 20.0; q, k, v of 2560 columns 10.1, now 5.9; weights in the cache: the
+// first 37.2, now 16.8, and Q4_K 9731 x 2560, q8_1, 7.1, now 5.2).
 #include "kq_device.h"
 #include "kq_items.h"
 #include "kq_launch.h"
@@ -171,10 +172,16 @@ struct XStage {
 // S lanes of a row take items s, s + S, ... in batches of N, all of a batch's
 // loads in flight at once; items past the row's end load the last one and
 // count as zero.
-template <class QT, int N, int RPS, int MODE>
+// SPAN: 64, a row takes the whole wave; 32, at most half of it; 0, either. A
+// kernel with both ways to sum a row costs a call of a few microseconds 0.05
+// to 0.2 us (quantizing, Q4_K 512 x 256: 2.73 us, apart 2.51; 2048 x 2048: 3.14
+// and 3.00); the launch of several matrices, which may hold both, loses with
+// kernels of their own (q, k and v of 4096 columns 6.7 -> 6.9 us).
+template <class QT, int N, int RPS, int MODE, int SPAN>
 __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_t rows, uint32_t cols, uint64_t rb,
                                           uint32_t log2s, const float *xf, const uint8_t *xq, float *__restrict__ y,
                                           uint32_t block, uint32_t nblocks, uint8_t *lds) {
+    if constexpr (SPAN == 64) log2s = 6;
     const uint32_t S = 1u << log2s;
     const uint32_t slots = WAVE >> log2s;
     const uint32_t lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, NW = blockDim.x / WAVE;
@@ -200,6 +207,10 @@ __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_
             }
         }
     };
+    // The matrix's arguments with x's, not in a second round trip behind x's
+    // loads: 0.05 us of the launch of several matrices (nothing with one, whose
+    // arguments are one cache line).
+    if constexpr (SPAN == 0) pin_args(w, rows, rb, log2s, nblocks);
     XStage<QT, MODE> xs;
     xs.load(xf, xq, cols);   // issued first: waiting for x then waits for nothing else
     // Neither the compiler nor the scheduler may move work across these two
@@ -234,7 +245,7 @@ __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_
         }
         i0 += N;
         if (S * i0 >= items) {   // the row group is done
-            if (log2s == 6) {
+            if (SPAN == 64 || (SPAN == 0 && log2s == 6)) {
                 // one row per wave instruction: the RPS rows reduce together
                 // (halving exchanges, no LDS); lane groups of 64 / RPS then
                 // hold row (lane >> SH) & (RPS - 1)
@@ -244,11 +255,27 @@ __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_
                 const uint32_t r = (lane >> SH) & (RPS - 1);
                 const uint32_t row = row_of(base, (int)r);
                 if ((lane & ((1u << SH) - 1)) == 0 && row < rows) y[row] = v;
+            } else if constexpr (SPAN == 32) {
+                auto sums = [&](auto g) {   // the lanes of a row slot sum on the VALU
+#pragma unroll
+                    for (int r = 0; r < RPS; r++) acc[r] = group_sum<decltype(g)::value>(acc[r]);
+                };
+                switch (log2s) {   // uniform
+                    case 5: sums(std::integral_constant<int, 32>{}); break;
+                    case 4: sums(std::integral_constant<int, 16>{}); break;
+                    case 3: sums(std::integral_constant<int, 8>{}); break;
+                    default: sums(std::integral_constant<int, 4>{}); break;
+                }
+#pragma unroll
+                for (int r = 0; r < RPS; r++) {
+                    const uint32_t row = row_of(base, r);
+                    if (s == 0 && row < rows) y[row] = acc[r];
+                }
             } else {
 #pragma unroll
                 for (int r = 0; r < RPS; r++) {
                     float v;
-                    switch (log2s) {   // uniform: the lanes of a row slot sum on the VALU
+                    switch (log2s) {   // uniform
                         case 5: v = group_sum<32>(acc[r]); break;
                         case 4: v = group_sum<16>(acc[r]); break;
                         case 3: v = group_sum<8>(acc[r]); break;
@@ -268,12 +295,12 @@ __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_
     }
 }
 
-template <class QT, int N, int RPS, int MODE>
+template <class QT, int N, int RPS, int MODE, int SPAN>
 __global__ void __launch_bounds__(GEMV_MAX_NT)
     k_gemv(const uint8_t *__restrict__ w, uint32_t rows, uint32_t cols, uint64_t rb, uint32_t log2s,
            const float *xf, const uint8_t *xq, float *__restrict__ y) {
     extern __shared__ __align__(16) uint8_t lds[];
-    gemv_rows<QT, N, RPS, MODE>(w, rows, cols, rb, log2s, xf, xq, y, blockIdx.x, gridDim.x, lds);
+    gemv_rows<QT, N, RPS, MODE, SPAN>(w, rows, cols, rb, log2s, xf, xq, y, blockIdx.x, gridDim.x, lds);
 }
 
 // Up to four GEMVs over one activation in one launch (the engine's
@@ -290,11 +317,11 @@ __global__ void __launch_bounds__(GEMV_MAX_NT) k_gemv_multi(GemvMultiArgs g) {
     const uint32_t start = m ? g.end[m - 1] : 0;
     const uint32_t blk = blockIdx.x - start, nblk = g.end[m] - start;
     if (g.type[m] == T_Q4_K)
-        gemv_rows<Q4K, N4, gemv_rps<Q4K>(N4), MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q4K::BB,
-                                                    g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q4K, N4, gemv_rps<Q4K>(N4), MODE, 0>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q4K::BB,
+                                                       g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
     else
-        gemv_rows<Q6K, N6, gemv_rps<Q6K>(N6), MODE>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q6K::BB,
-                                                    g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q6K, N6, gemv_rps<Q6K>(N6), MODE, 0>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q6K::BB,
+                                                       g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
 }
 
 // How a row's items are spread: S lanes (a power of two) take N items each
@@ -388,7 +415,7 @@ static hipError_t gemv_dispatch(const uint8_t *w, uint64_t rows, uint64_t cols, 
         const GemvGrid gg = gemv_grid(waves, cols, cus);
         const uint64_t iters = (waves + gg.nw - 1) / gg.nw, cap = (uint64_t)gg.cap * cus;
         const uint32_t grid = (uint32_t)(iters < cap ? iters : cap);
-        auto kern = k_gemv<QT, N, RPS, MODE>;
+        auto kern = sh.S == 64 ? k_gemv<QT, N, RPS, MODE, 64> : k_gemv<QT, N, RPS, MODE, 32>;
         const hipError_t e = lds_limit(kern, lds);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * gg.nw), lds, st, w, (uint32_t)rows, (uint32_t)cols, rb,
