@@ -447,6 +447,21 @@ static hipError_t gemv_multi_dispatch(GemvMultiArgs &g, int n, const uint64_t *r
     // q, k and v of 4096 columns take 6.6 us in 4 waves, 8.3 in 6, 7.6 in 8.
     GemvGrid gg{4, 8};
     if (total > 16ull * cus) gg = gemv_grid(total, g.cols, cus);
+    // From 16 to 64 waves per CU and up to 5120 columns: the workgroups whose
+    // last round leaves the busiest CU the fewest waves, the fewest workgroups
+    // among equals (quantizing, q, k and v of 4096 rows and columns: 768
+    // workgroups of 8 waves are three per CU, 9.1 us, and a round and a half of
+    // two per CU, 10.4; of 5120: 6 waves, three per CU, 16.6 and 18.8). At 6144
+    // columns the third staging of the activation costs what it gains (Q4_K,
+    // 6144 and twice 1536 rows 11.2 against 10.2 us).
+    if (total > 16ull * cus && total <= 64ull * cus && g.cols > 2048 && g.cols <= 5120) {
+        uint64_t best = ~0ull;
+        for (const GemvGrid c : {GemvGrid{8, 2}, GemvGrid{6, 3}, GemvGrid{8, 4}}) {
+            const uint64_t wgs = (total + c.nw - 1) / c.nw, slots = (uint64_t)c.cap * cus;
+            const uint64_t busiest = c.nw * (wgs <= slots ? (wgs + cus - 1) / cus : c.cap * ((wgs + slots - 1) / slots));
+            if (busiest < best) gg = c, best = busiest;
+        }
+    }
     total = 0;
     for (int i = 0; i < n; i++) {   // waves -> workgroups
         iters[i] = (iters[i] + gg.nw - 1) / gg.nw;
