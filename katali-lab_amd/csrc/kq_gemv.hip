@@ -332,8 +332,8 @@ __global__ void __launch_bounds__(GEMV_MAX_NT) k_gemv_multi(GemvMultiArgs g) {
 // a chain and a small matrix more waves (Q4_K 9731 x 2560, 32 lanes x 3
 // items: 5.6 us, 16 x 5: 6.4; 5120 x 5120 6.5 and 7.7). A large matrix fills
 // the chip either way and pays for the padding instead, so there at most an
-// eighth comes first (Q4_K 20000 x 5120, 64 x 3: 14.5 us, 32 x 5: 13.0; Q6_K
-// 40000 x 5120 37.4 and 34.2).
+// eighth comes first (q8_1 and weights from memory: Q4_K 20000 x 5120, 64 x 3:
+// 13.7 us, 32 x 5: 12.5; Q6_K 40000 x 5120 35.7 and 33.2).
 struct GemvShape {
     uint32_t S, N;
 };
@@ -360,11 +360,13 @@ constexpr GemvShapes gemv_shapes() {
 }
 template <class QT>
 inline constexpr GemvShapes GEMV_SHAPES = gemv_shapes<QT>();
-// large: from 6144 items per CU (between 0.8 and 2.4 million measured)
+// large: from 10240 items per CU, 2.6 million (the least padded spread loses
+// up to 2.2 million, Q4_K 18944 x 3584 10.6 against 9.3 us, Q6_K 20000 x 5120
+// 20.8 against 19.8, 28000 x 5120 26.6 against 25.8, and wins from 3.2 million)
 template <class QT>
 constexpr GemvShape gemv_shape(uint64_t rows, uint64_t cols, uint64_t cus) {
     const uint64_t nb = cols / 256;
-    return GEMV_SHAPES<QT>.s[nb][rows * nb * QT::IPB > 6144 * cus];
+    return GEMV_SHAPES<QT>.s[nb][rows * nb * QT::IPB > 10240 * cus];
 }
 // the item counts that the two formats have at one and the same row length
 constexpr bool gemv_pair(uint32_t n4, uint32_t n6) {
