@@ -403,6 +403,17 @@ static GemvGrid gemv_grid(uint64_t waves, uint64_t cols, uint32_t cus) {
     return best;
 }
 
+// No more workgroups per CU than their activation leaves room for: an fp32 one
+// takes 4.75 bytes a column, from 16640 columns more than half of the LDS, and
+// the second half of the grid would queue and stage it again (weights from
+// memory, Q6_K 4096 x 16640 22.8 against 18.3 us, Q4_K 8192 x 28672 42.4
+// against 36.6).
+static GemvGrid lds_fit(GemvGrid g, uint32_t lds) {
+    const uint32_t most = LDS_PER_WG / lds;
+    if (g.cap > most) g.cap = most;
+    return g;
+}
+
 template <class QT, int MODE>
 static hipError_t gemv_dispatch(const uint8_t *w, uint64_t rows, uint64_t cols, const float *xf, const uint8_t *xq,
                                 float *y, hipStream_t st) {
@@ -414,7 +425,7 @@ static hipError_t gemv_dispatch(const uint8_t *w, uint64_t rows, uint64_t cols, 
         constexpr int N = decltype(n)::value, RPS = gemv_rps<QT>(N);
         const uint32_t rows_per_wave = 64 / sh.S * RPS;
         const uint64_t waves = (rows + rows_per_wave - 1) / rows_per_wave;
-        const GemvGrid gg = gemv_grid(waves, cols, cus);
+        const GemvGrid gg = lds_fit(gemv_grid(waves, cols, cus), lds);
         const uint64_t iters = (waves + gg.nw - 1) / gg.nw, cap = (uint64_t)gg.cap * cus;
         const uint32_t grid = (uint32_t)(iters < cap ? iters : cap);
         auto kern = sh.S == 64 ? k_gemv<QT, N, RPS, MODE, 64> : k_gemv<QT, N, RPS, MODE, 32>;
@@ -469,7 +480,7 @@ static hipError_t gemv_multi_dispatch(GemvMultiArgs &g, int n, const uint64_t *r
         iters[i] = (iters[i] + gg.nw - 1) / gg.nw;
         total += iters[i];
     }
-    const uint64_t cap = (uint64_t)gg.cap * cus;
+    const uint64_t cap = (uint64_t)lds_fit(gg, lds).cap * cus;
     uint32_t end = 0;
     for (int i = 0; i < GEMV_MULTI_MAX; i++) {
         if (i < n) {
