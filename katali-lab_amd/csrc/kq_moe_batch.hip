@@ -61,9 +61,10 @@ __host__ __device__ inline uint32_t mb_small_off() { return 16; }
 __host__ __device__ inline uint32_t mb_big_off(uint32_t P) { return mb_small_off() + GRP_REC * P; }
 static_assert(MB_REC % 4 == 0 && GRP_REC % 4 == 0, "entry records: whole int4s");
 static_assert(GRP_REC == 4 + MB_GRP, "small entries: the pairs inline");
-// Past the small records: entry indices up to the grid's (P / 8 + one per
-// expert, above P only when P is below the expert count) read their record
-// before they know that they have none.
+// A small entry's workgroups read their record before they know whether the
+// list has it, and the grid has up to P + P / 8 entries: the records read past
+// the list's P lie in the grouped-GEMM records behind it.
+static_assert(GRP_REC <= MB_GRP * MB_REC, "P / 8 small records fit the P grouped-GEMM records behind the list");
 uint64_t moe_batch_meta_words(uint32_t P) { return mb_big_off(P) + MB_REC * P; }
 
 // Inclusive prefix sum over the 64 lanes of a wave on the VALU: row_shr 1, 2,
@@ -789,7 +790,8 @@ hipError_t launch_moe_batch(const MoeArgs &base, uint32_t T, uint32_t min_big, c
     a.bS = S;
     a.bslot = meta + mb_small_off();
     a.bcount = meta;
-    // small entries: at most P / 8 + one per expert (each has >= 1 pair)
+    // small entries: at most P / 8 + one per expert (each has >= 1 pair), so
+    // never above P + P / 8 (moe_batch_meta_words)
     const uint32_t ne = base.n_expert + 1;
     const uint32_t max_small = P / MB_GRP + (ne < P ? ne : P);
     // No expert can reach min_big pairs below min_big pairs in all: then the
