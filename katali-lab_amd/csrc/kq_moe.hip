@@ -3062,9 +3062,12 @@ static hipError_t go_a(const MoeArgs &a, uint32_t n_slots, hipStream_t s, bool m
     if (NORMED && L.scl + normed_area_bytes(a.hidden) > lds) lds = L.scl + normed_area_bytes(a.hidden);
     if constexpr (!NORMED && NB >= 8) {   // hidden 2048 and 4096
         // Routed layers too at hidden 4096 (8-wave workgroups, two per CU: 288
-        // units 17.4 -> 15.3 us, 896 units 31.3 -> 30.4); at 2048 a half unit
-        // is 16 waves that route for half the rows, and loses (320 units 10.2
-        // -> 14.0 us).
+        // units 17.4 -> 15.3 us, 896 units 31.3 -> 30.4; layers of 288 to 896
+        // units in 2 to 10 slots gain 1.9 to 2.4 us); at 2048 a half unit is 16
+        // waves that route for half the rows, and loses (layers of 272 to 896
+        // units in 2 to 12 slots take 1.4 to 5.2 us more). The half kernel is
+        // built with two keys a lane, so routed layers of more than 128 experts
+        // keep whole units.
         if (may_wait && !xcd_disabled() && (a.n_sel == 0 || (NB == 16 && a.n_expert <= 128)) && a.fsync &&
             half_units(units, (uint32_t)device_cu_count()) && units <= DH_MAX_BLOCKS && !env_half_off()) {
             hipLaunchKernelGGL((k_moe_gu<NB, 2, false, true>), dim3(2 * units), dim3(a1_threads<NB>()),

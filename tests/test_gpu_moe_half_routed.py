@@ -110,3 +110,63 @@ def test_half_units_off_where_nothing_waits(hip, monkeypatch, ffn, n_exp, k, sha
         hip.one_launch(1)
     for _ in range(3):
         assert np.array_equal(run(), ref)
+
+
+# ffn, experts (all selected), half units: 896 units are the most on 256 CUs
+# that half units split more evenly; 1056 split so too, but pass the 1024
+# counters of the exchange and stay whole
+MANY = [(14336, 2, True), (8448, 4, False)]
+
+
+@pytest.mark.parametrize("ffn,k,halves", MANY)
+def test_half_units_many_blocks(hip, oracle, monkeypatch, ffn, k, halves):
+    """Counters and tagged words of high block numbers, in the library's
+    exchange area and in the allocation-free entry's own."""
+    import katali_hip as K
+    print(f"[moe_half_many] ffn={ffn} k={k}", flush=True)
+    hidden, units = 4096, k * ffn // 32
+    bufs = []
+    for t, r, c in ((Q4_K, ffn, hidden), (Q4_K, ffn, hidden), (Q6_K, hidden, ffn)):
+        nb = k * r * (c // 256)
+        bufs.append(hip.alloc(nb * K.BLOCK_BYTES[t]))
+        hip.synth_fill(t, bufs[-1], nb, k + r + t)
+    desc = hip.moe_desc(hidden, ffn, k, *bufs, down_type=Q6_K)
+    rng = np.random.default_rng(ffn)
+    x = hip.to_device(S.activation(rng, hidden))
+    route = hip.moe_route(k, logits=hip.to_device(rng.standard_normal(k).astype(np.float32)))
+    y, gu, hq = hip.alloc(hidden * 4), hip.alloc(k * 2 * ffn * 4), hip.alloc(units * 36)
+
+    def run():
+        for _ in range(3):
+            hip.moe_layer_debug(desc, route, y, gu, hq, x=x)
+        hip.sync()
+        return y.download(np.uint32), gu.download(np.uint32), hq.download(np.uint8)
+    monkeypatch.setenv("KATALI_HIP_HALF_UNITS", "0")
+    want = run()
+    monkeypatch.delenv("KATALI_HIP_HALF_UNITS")
+    for a, b, what in zip(want, run(), ("y", "gate/up", "h blocks")):
+        assert np.array_equal(a, b), what
+    h = hq.download(np.uint8).reshape(units, 36)
+    gq = gu.download(np.float32).reshape(k, 2, ffn)
+    assert np.isfinite(gq).all() and h[:, 4:].any(axis=1).all()   # every block was written
+    hip.graph_begin()
+    hip.moe_layer_noalloc(desc, route, y, x=x)
+    gr = hip.graph_end()
+    try:
+        for rep in range(3):
+            for entry in (hip.moe_layer, hip.moe_layer_noalloc, None):
+                hip.memset(y, 0, hidden * 4)
+                hip.graph_launch(gr) if entry is None else entry(desc, route, y, x=x)
+                hip.sync()
+                assert np.array_equal(y.download(np.uint32), want[0]), (rep, entry)
+    finally:
+        hip.graph_destroy(gr)
+    if halves:   # the hook sets block 0's counter off: half units did run if a wait expires
+        monkeypatch.setenv("KATALI_HIP_TEST_SKEW", "1")
+        try:
+            with pytest.raises(K.HipError) as err:
+                hip.moe_layer(desc, route, y, x=x)
+                hip.sync()   # clears the exchange area
+            assert err.value.rc == K.E_TIMEOUT, err.value
+        finally:
+            hip.one_launch(1)

@@ -8,7 +8,9 @@ of a 256-CU device, with the occupancy API reporting at least one block of
 the kernel per CU (launch_moe_xcd and launch_moe_stack).
 
 The wide down projection's plan: every shape that the layer's LDS rule admits
-has one, on any CU count, within the LDS, its row index exact."""
+has one, on any CU count, within the LDS, its row index exact.
+
+Kernel A's half units: where the busiest CU has less work with them."""
 import os
 import subprocess
 
@@ -59,6 +61,17 @@ int main() {
 """
 
 
+HALF_DRIVER = r"""
+#include <stdio.h>
+#include "kq_plan.h"
+int main() {
+    for (unsigned u = 8; u <= 1160; u++)
+        if (kq::half_units(u, 256)) printf("%u\n", u);
+    return 0;
+}
+"""
+
+
 def run_driver(tmp_path, code):
     src = tmp_path / "plan.cpp"
     src.write_text(code)
@@ -80,3 +93,10 @@ def test_coresident_rule(tmp_path):
     # one per CU on exactly 256 CUs: yes; a kernel that fits no CU, another
     # CU count (the slot-to-XCD mapping needs 256), a grid above the CUs: no
     assert out == ["1", "1", "0", "0", "0", "0", "0", "1", "0"]
+
+
+def test_half_units_rule(tmp_path):
+    got = list(map(int, run_driver(tmp_path, HALF_DRIVER)))
+    # whole workgroups of eight units, in the lower half of each round of CUs
+    want = [u for u in range(8, 1161) if u % 8 == 0 and (0 < u % 256 <= 128)]
+    assert got == want and 896 in got and 1056 in got and not any(896 < u <= 1024 for u in got)
