@@ -1,6 +1,7 @@
 """Kernel B for long down rows: every split of a pair's items on lanes (16, 32
-and 64 lanes, whole and padded), more slots than waves, ragged row runs,
-and a shape whose h does not fit its layout (kernel B's loop takes it).
+and 64 lanes, whole and padded), more slots than waves, runs of 1 to 8 rows per
+workgroup and h up to the LDS limit. (Runs that do not divide the rows need
+another CU count than the device's: tests/test_plan_rules.py checks their plans.)
 
 The down projection alone is compared: the oracle's from the GPU's own h
 blocks, so the difference is the order of fp32 sums (1e-5 as in the layer's
@@ -28,7 +29,9 @@ CASES = [
     (512, 13824, 3, 2, False, Q6_K),
     (256, 16384, 2, 1, False, Q6_K),     # the longest rows
     (256, 16384, 2, 1, False, Q4_K),
-    (256, 14336, 8, 8, False, Q4_K),     # h past the LDS in item order
+    (256, 14336, 8, 8, False, Q4_K),     # h near the LDS limit
+    (4096, 4352, 2, 2, False, Q6_K),     # 8 rows per workgroup
+    (4096, 4608, 2, 2, True, Q4_K),
 ]
 
 
