@@ -346,7 +346,7 @@ int katali_hip_moe_check(const KataliHipMoe *moe, int32_t n_sel, uint32_t n_toke
  * one-launch layer where that entry takes it, under the same environment
  * switches), so its results are bit-identical to it. Its routing hand-off,
  * q8_1 h blocks and the one-launch layer's exchange words live in a fixed
- * static device array of the library (one per GPU, about 590 KB, held until
+ * static device array of the library (one per GPU, about 820 KB, held until
  * the process ends): n_slots * ffn/32 * 36 bytes of h must fit 135168
  * (n_slots = n_sel + 1 with a shared expert), else KATALI_HIP_E_INVALID;
  * every shape that passes katali_hip_moe_check's LDS rule needs at most
