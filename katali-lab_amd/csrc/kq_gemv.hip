@@ -177,7 +177,7 @@ struct XStage {
 // to 0.2 us (quantizing, Q4_K 512 x 256: 2.73 us, apart 2.51; 2048 x 2048: 3.14
 // and 3.00); the launch of several matrices, which may hold both, loses with
 // kernels of their own (q, k and v of 4096 columns 6.7 -> 6.9 us).
-template <class QT, int N, int RPS, int MODE, int SPAN>
+template <class QT, int N, int RPS, int MODE, int SPAN, bool PIN = false>
 __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_t rows, uint32_t cols, uint64_t rb,
                                           uint32_t log2s, const float *xf, const uint8_t *xq, float *__restrict__ y,
                                           uint32_t block, uint32_t nblocks, uint8_t *lds) {
@@ -208,9 +208,8 @@ __device__ __forceinline__ void gemv_rows(const uint8_t *__restrict__ w, uint32_
         }
     };
     // The matrix's arguments with x's, not in a second round trip behind x's
-    // loads: 0.05 us of the launch of several matrices (nothing with one, whose
-    // arguments are one cache line).
-    if constexpr (SPAN == 0) pin_args(w, rows, rb, log2s, nblocks);
+    // loads (gemv_multi_pin; one matrix's arguments are one cache line).
+    if constexpr (PIN) pin_args(w, rows, rb, log2s, nblocks);
     XStage<QT, MODE> xs;
     xs.load(xf, xq, cols);   // issued first: waiting for x then waits for nothing else
     // Neither the compiler nor the scheduler may move work across these two
@@ -303,6 +302,15 @@ __global__ void __launch_bounds__(GEMV_MAX_NT)
     gemv_rows<QT, N, RPS, MODE, SPAN>(w, rows, cols, rb, log2s, xf, xq, y, blockIdx.x, gridDim.x, lds);
 }
 
+// Where the launch of several matrices reads a matrix's arguments ahead of x's
+// loads: up to 2048 columns and quantizing up to 4096, by Q4_K's items a lane
+// (weights from memory, without and with: quantizing, q, k and v of 512 columns
+// 3.39 -> 3.32 us, of 4096 6.75 -> 6.70). For longer rows x's loads behind one
+// more wait cost what it gains or more (fp32 4096 6.72 and 6.76, quantizing 3072
+// 5.66 and 5.72).
+template <int N4, int MODE>
+constexpr bool gemv_multi_pin() { return N4 == 1 || (MODE == 2 && N4 == 2); }
+
 // Up to four GEMVs over one activation in one launch (the engine's
 // matvec_multi: q, k and v of a layer). Matrix m owns workgroups
 // [end[m-1], end[m]) and runs the single-matrix body on them, so each row's
@@ -316,12 +324,15 @@ __global__ void __launch_bounds__(GEMV_MAX_NT) k_gemv_multi(GemvMultiArgs g) {
         if (blockIdx.x >= g.end[i]) m = i + 1;   // end[] is non-decreasing, padded with the total
     const uint32_t start = m ? g.end[m - 1] : 0;
     const uint32_t blk = blockIdx.x - start, nblk = g.end[m] - start;
+    constexpr bool PIN = gemv_multi_pin<N4, MODE>();
     if (g.type[m] == T_Q4_K)
-        gemv_rows<Q4K, N4, gemv_rps<Q4K>(N4), MODE, 0>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q4K::BB,
-                                                       g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q4K, N4, gemv_rps<Q4K>(N4), MODE, 0, PIN>(g.w[m], g.rows[m], g.cols,
+                                                            (uint64_t)(g.cols / 256) * Q4K::BB, g.log2s[m], g.x, nullptr,
+                                                            g.y[m], blk, nblk, lds);
     else
-        gemv_rows<Q6K, N6, gemv_rps<Q6K>(N6), MODE, 0>(g.w[m], g.rows[m], g.cols, (uint64_t)(g.cols / 256) * Q6K::BB,
-                                                       g.log2s[m], g.x, nullptr, g.y[m], blk, nblk, lds);
+        gemv_rows<Q6K, N6, gemv_rps<Q6K>(N6), MODE, 0, PIN>(g.w[m], g.rows[m], g.cols,
+                                                            (uint64_t)(g.cols / 256) * Q6K::BB, g.log2s[m], g.x, nullptr,
+                                                            g.y[m], blk, nblk, lds);
 }
 
 // How a row's items are spread: S lanes (a power of two) take N items each
