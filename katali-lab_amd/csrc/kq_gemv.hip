@@ -374,11 +374,13 @@ template <class QT>
 inline constexpr GemvShapes GEMV_SHAPES = gemv_shapes<QT>();
 // large: from 10240 items per CU, 2.6 million (the least padded spread loses
 // up to 2.2 million, Q4_K 18944 x 3584 10.6 against 9.3 us, Q6_K 20000 x 5120
-// 20.8 against 19.8, 28000 x 5120 26.6 against 25.8, and wins from 3.2 million)
+// 20.8 against 19.8, 28000 x 5120 26.6 against 25.8, and wins from 3.2 million);
+// from 6144, 1.6 million, with Q6_K up to 4096 columns, whose least padded rows
+// run in workgroups of 4 waves (gemv_grid; 40000 x 2560 18.2 against 19.7).
 template <class QT>
 constexpr GemvShape gemv_shape(uint64_t rows, uint64_t cols, uint64_t cus) {
-    const uint64_t nb = cols / 256;
-    return GEMV_SHAPES<QT>.s[nb][rows * nb * QT::IPB > 10240 * cus];
+    const uint64_t nb = cols / 256, line = QT::TYPE == T_Q6_K && cols <= 4096 ? 6144 : 10240;
+    return GEMV_SHAPES<QT>.s[nb][rows * nb * QT::IPB > line * cus];
 }
 // the item counts that the two formats have at one and the same row length
 constexpr bool gemv_pair(uint32_t n4, uint32_t n6) {
@@ -388,31 +390,55 @@ constexpr bool gemv_pair(uint32_t n4, uint32_t n6) {
 }
 
 // Waves per workgroup and the most workgroups per CU, for `waves` waves of
-// rows. Up to 16 waves per CU: the count (4, 6 or 8) that puts the fewest
-// waves on the busiest CU, which sets the time, the largest among equals
-// (fewer workgroups stage the activation): 6144 rows of 2048 columns in 6
-// waves make 256 workgroups, one per CU; 4096 x 4096 Q4_K takes 4.3 us in 256
-// workgroups of 8 waves, 4.9 in 512 of 4. Past that the workgroups loop over
-// their rows: above 2048 columns two resident ones of 8 waves, so that the
-// activation is staged twice per CU rather than once per 4 waves (Q6_K 5120 x
-// 13824: 20.3 against 26.0 us; Q4_K 9731 x 2560: 6.0 against 6.8), up to there
-// as many of 4 waves as fit (Q4_K 25000 x 1536: 6.5 against 7.1 us in 8
-// waves). Past 64 waves per CU each loops many times and four of 8 waves
-// keep more loads in flight (Q4_K 40000 x 4096: 22.9 against 23.5 us in two).
+// rows; the busiest CU, with the most of them, sets the time. us with q8_1 and
+// weights from memory where nothing else is said:
+//   - up to 4 waves per CU 4 (no count puts fewer on a CU);
+//   - up to 16 the count (4, 6 or 8) that puts the fewest on the busiest CU.
+//     Among equals 8 (fewer workgroups stage the activation: Q4_K 4096 x 4096
+//     4.3 in 256 workgroups of 8 waves, 4.9 in 512 of 4), but 4 rather than 6 up
+//     to 4096 columns, quantizing up to 2048 (Q4_K 6144 x 4096 5.0 and 5.5,
+//     11008 x 2048 4.6 and 5.1), and 4 rather than 8 for Q6_K from 2048 to 4096
+//     columns and up to 14 waves (14336 x 2560 9.1 and 9.5);
+//   - above, workgroups that loop over their rows: two of 8 waves, so that the
+//     activation is staged twice per CU rather than once per 4 waves (Q6_K 5120
+//     x 13824, fp32: 20.3 against 26.0; Q4_K 9731 x 2560: 6.0 against 6.8), and
+//     up to 2048 columns as many of 4 as fit (Q4_K 25000 x 1536: 6.5 against
+//     7.1), unless they quantize for Q4_K in more than one round (40000 x 2048:
+//     9.5 in two of 8, 11.1). With Q6_K up to 4096 columns and 32 waves
+//     (quantizing 20) of 4 too where the busiest CU gets fewer (20000 x 2560:
+//     11.0 and 12.6), of batches of five items four (their registers);
+//   - past 64 waves per CU each loops many times and four of 8 waves keep more
+//     loads in flight (Q4_K 40000 x 4096, fp32: 22.9 against 23.5 in two).
+// One of 8 waves, which stages the activation once, where that is most of a
+// workgroup's work: quantizing for Q4_K rows of a whole wave from 8 to 16 waves
+// per CU (6144 x 4096: 5.5, in two of 6 waves 6.2), and Q6_K rows of four items a
+// lane and more from 8 to 32, but not with fp32 (4096 x 14336: 14.0 and 15.7).
 struct GemvGrid {
     uint32_t nw, cap;
 };
-static GemvGrid gemv_grid(uint64_t waves, uint64_t cols, uint32_t cus) {
-    if (waves <= 4ull * cus) return {4, 8};   // no count puts fewer than 4 on a CU
-    if (waves > 64ull * cus) return {8, 4};
-    if (waves > 16ull * cus) return cols > 2048 ? GemvGrid{8, 2} : GemvGrid{4, 8};
-    GemvGrid best{4, 8};
-    uint64_t best_waves = ~0ull;
-    for (uint32_t nw : {4u, 6u, 8u}) {
-        const uint64_t busiest = ((waves + nw - 1) / nw + cus - 1) / cus * nw;
-        if (busiest <= best_waves) best.nw = nw, best_waves = busiest;
+template <class QT, int MODE>
+static GemvGrid gemv_grid(GemvShape sh, uint64_t waves, uint64_t cols, uint32_t cus) {
+    constexpr bool Q6 = QT::TYPE == T_Q6_K, QUANT = MODE == 2;
+    auto upto = [&](uint64_t per_cu) { return waves <= per_cu * cus; };
+    auto busiest = [&](uint32_t nw) { return ((waves + nw - 1) / nw + cus - 1) / cus * nw; };
+    if (upto(4)) return {4, 8};
+    if (!upto(64)) return {8, 4};
+    if (sh.S == 64 && !upto(8)) {
+        if (Q6 && MODE != 0 && sh.N >= 4 && upto(32)) return {8, 1};
+        if (!Q6 && QUANT && cols > 2048 && upto(16)) return {8, 1};
     }
-    return best;
+    const uint64_t b4 = busiest(4), b6 = busiest(6), b8 = busiest(8);
+    if (upto(16)) {
+        const bool four = b4 <= b6 && b4 <= b8 && !upto(8) && cols <= (QUANT ? 2048 : 4096);
+        if (four && (b4 < b8 || (Q6 && cols > 2048 && upto(14)))) return {4, 8};
+        return b8 <= b4 && b8 <= b6 ? GemvGrid{8, 2} : (b6 <= b4 ? GemvGrid{6, 3} : GemvGrid{4, 8});
+    }
+    if (cols <= 2048) return !Q6 && QUANT && !upto(32) && b4 >= b8 ? GemvGrid{8, 2} : GemvGrid{4, 8};
+    if (Q6 && cols <= 4096) {
+        if (sh.N == 5 && upto(32)) return {4, 4};
+        if (b4 < b8 && upto(QUANT ? 20 : 32)) return {4, 8};
+    }
+    return {8, 2};
 }
 
 // No more workgroups per CU than their activation leaves room for: an fp32 one
@@ -437,7 +463,7 @@ static hipError_t gemv_dispatch(const uint8_t *w, uint64_t rows, uint64_t cols, 
         constexpr int N = decltype(n)::value, RPS = gemv_rps<QT>(N);
         const uint32_t rows_per_wave = 64 / sh.S * RPS;
         const uint64_t waves = (rows + rows_per_wave - 1) / rows_per_wave;
-        const GemvGrid gg = lds_fit(gemv_grid(waves, cols, cus), lds);
+        const GemvGrid gg = lds_fit(gemv_grid<QT, MODE>(sh, waves, cols, cus), lds);
         const uint64_t iters = (waves + gg.nw - 1) / gg.nw, cap = (uint64_t)gg.cap * cus;
         const uint32_t grid = (uint32_t)(iters < cap ? iters : cap);
         auto kern = sh.S == 64 ? k_gemv<QT, N, RPS, MODE, 64> : k_gemv<QT, N, RPS, MODE, 32>;
@@ -471,17 +497,19 @@ static hipError_t gemv_multi_dispatch(GemvMultiArgs &g, int n, const uint64_t *r
     // The matrices' workgroups differ in work, and small ones even that out:
     // q, k and v of 4096 columns take 6.6 us in 4 waves, 8.3 in 6, 7.6 in 8.
     GemvGrid gg{4, 8};
-    if (total > 16ull * cus) gg = gemv_grid(total, g.cols, cus);
+    if (total > 64ull * cus) gg = {8, 4};
+    else if (total > 16ull * cus && g.cols > 2048) gg = {8, 2};
     // From 16 to 64 waves per CU and up to 5120 columns: the workgroups whose
     // last round leaves the busiest CU the fewest waves, the fewest workgroups
     // among equals (quantizing, q, k and v of 4096 rows and columns: 768
     // workgroups of 8 waves are three per CU, 9.1 us, and a round and a half of
-    // two per CU, 10.4; of 5120: 6 waves, three per CU, 16.6 and 18.8). At 6144
-    // columns the third staging of the activation costs what it gains (Q4_K,
-    // 6144 and twice 1536 rows 11.2 against 10.2 us).
+    // two per CU, 10.4; of 5120: 6 waves, three per CU, 16.6 and 18.8), but
+    // quantizing three per CU rather than two (4096 rows of 5120 columns 13.9
+    // and 15.3). At 6144 columns the third staging of the activation costs what
+    // it gains (Q4_K, 6144 and twice 1536 rows 11.2 against 10.2 us).
     if (total > 16ull * cus && total <= 64ull * cus && g.cols > 2048 && g.cols <= 5120) {
         uint64_t best = ~0ull;
-        for (const GemvGrid c : {GemvGrid{8, 2}, GemvGrid{6, 3}, GemvGrid{8, 4}}) {
+        for (const GemvGrid c : {GemvGrid{8, MODE == 2 ? 3u : 2u}, GemvGrid{8, 2}, GemvGrid{6, 3}, GemvGrid{8, 4}}) {
             const uint64_t wgs = (total + c.nw - 1) / c.nw, slots = (uint64_t)c.cap * cus;
             const uint64_t busiest = c.nw * (wgs <= slots ? (wgs + cus - 1) / cus : c.cap * ((wgs + slots - 1) / slots));
             if (busiest < best) gg = c, best = busiest;
