@@ -78,3 +78,68 @@ def test_gemv_multi_large_and_small(hip):
                 one = hip.alloc(r * 4)
                 (hip.matvec_dp4a if dp4a else hip.matvec)(t, wd, r, cols, xd, one)
                 assert np.array_equal(y.download(np.uint32), one.download(np.uint32))
+
+
+# The workgroups that gemv_grid picks on 256 CUs, by waves per CU
+GRIDS = [
+    (Q4_K, 6143, 4096),    # 12: workgroups of 4 waves; quantizing one of 8 per CU
+    (Q4_K, 11001, 2048),   # 10.7: of 4 waves
+    (Q4_K, 40003, 2048),   # 39: as many of 4 as fit; quantizing two of 8
+    (Q6_K, 14333, 2560),   # 14: of 4 waves; quantizing two of 8
+    (Q6_K, 20003, 2560),   # 19.5: of 4 waves past 16
+    (Q6_K, 25603, 3072),   # 25: of 4 waves; quantizing two of 8
+    (Q6_K, 40003, 2560),   # the least padded spread, four of 4 waves
+    (Q6_K, 2501, 14336),   # 9.8: one of 8 waves; fp32 two of 6
+    (Q6_K, 5633, 20480),   # 22: the same with five items a lane
+]
+
+
+@pytest.mark.parametrize("t,rows,cols", GRIDS, ids=[f"{'q4k' if s[0] == Q4_K else 'q6k'}_{s[1]}x{s[2]}" for s in GRIDS])
+def test_gemv_workgroups(hip, t, rows, cols):
+    """Every row has the bits it has in a launch of few rows (up to 4 waves per
+    CU), however the workgroups share them. At 40003 x 2560 the spread differs
+    too, so there the order of the fp32 sums differs (1e-5 as above)."""
+    print(f"[gemv_workgroups] type={t} rows={rows} cols={cols}", flush=True)
+    rb, few = cols // 256 * (144 if t == Q4_K else 210), 1000
+
+    class At:   # rows from `first` on
+        def __init__(self, buf, first):
+            self.ptr = buf.ptr + first * rb
+    xd, xqd = hip.alloc(cols * 4), hip.alloc(cols // 32 * 36)
+    hip.synth_normal(xd, cols, 3)
+    hip.quantize_q8_1(xd, cols, xqd)
+    wd = hip.alloc(rows * rb)
+    hip.synth_fill(t, wd, rows * cols // 256, rows)
+    y, part = hip.alloc((rows + 1) * 4), hip.alloc(few * 4)
+    for call, x in ((hip.matvec, xd), (hip.matvec_dp4a, xd), (hip.matvec_q8, xqd)):
+        y.upload(np.full(rows + 1, 7.25, np.float32))
+        call(t, wd, rows, cols, x, y)
+        got = y.download(np.float32)
+        assert got[rows] == 7.25
+        for r0 in range(0, rows, few):
+            n = min(few, rows - r0)
+            call(t, At(wd, r0), n, cols, x, part)
+            want = part.download(np.float32, n)
+            if (t, rows, cols) == (Q6_K, 40003, 2560):
+                assert np.linalg.norm(got[r0:r0 + n] - want) <= 1e-5 * np.linalg.norm(want), r0
+            else:
+                assert np.array_equal(got[r0:r0 + n].view(np.uint32), want.view(np.uint32)), (call.__name__, r0)
+
+
+def test_gemv_multi_three_per_cu(hip):
+    """Quantizing, 38 waves per CU: three workgroups of 8 waves, which loop."""
+    print("[gemv_multi_three_per_cu]", flush=True)
+    cols, mats = 5120, [(Q4_K, 8191), (Q4_K, 1023), (Q6_K, 1021)]
+    xd = hip.alloc(cols * 4)
+    hip.synth_normal(xd, cols, 5)
+    wds = [hip.alloc(r * cols // 256 * (144 if t == Q4_K else 210)) for t, r in mats]
+    for i, ((t, r), wd) in enumerate(zip(mats, wds)):
+        hip.synth_fill(t, wd, r * cols // 256, 60 + i)
+    ys = [hip.alloc((r + 1) * 4) for _, r in mats]
+    for (t, r), y in zip(mats, ys):
+        y.upload(np.full(r + 1, 7.25, np.float32))
+    hip.matvec_multi([t for t, _ in mats], wds, [r for _, r in mats], cols, xd, ys, dp4a=True)
+    for (t, r), wd, y in zip(mats, wds, ys):
+        one, got = hip.alloc(r * 4), y.download(np.float32)
+        hip.matvec_dp4a(t, wd, r, cols, xd, one)
+        assert got[r] == 7.25 and np.array_equal(got[:r].view(np.uint32), one.download(np.uint32))
