@@ -61,13 +61,13 @@ __device__ __forceinline__ Best block_best(Best b) {
 }
 
 constexpr uint32_t ARGMAX_PARTS = 256;
-constexpr uint32_t ARGMAX_U = 4;
 constexpr uint32_t ARGMAX_COUNT = 2 * ARGMAX_PARTS;   // the count word, after the partials
 
 __device__ __forceinline__ uint64_t pack(Best b) { return ((uint64_t)(uint32_t)b.i << 32) | __float_as_uint(b.v); }
 __device__ __forceinline__ Best unpack(uint64_t w) { return Best{__uint_as_float((uint32_t)w), (int32_t)(w >> 32)}; }
 
 // words: ARGMAX_PARTS 64-bit partials, then the count (zero between calls)
+template <uint32_t ARGMAX_U>
 __global__ void __launch_bounds__(256) k_argmax(const float *__restrict__ x, uint32_t n, uint32_t *words,
                                                 int32_t *out) {
     __shared__ uint32_t last;
@@ -106,11 +106,17 @@ __global__ void __launch_bounds__(256) k_argmax(const float *__restrict__ x, uin
 uint32_t argmax_scratch_bytes() { return 4 * (ARGMAX_COUNT + 1); }
 
 hipError_t launch_argmax(const float *x, uint32_t n, void *scratch, int32_t *out, hipStream_t s) {
-    uint32_t g = (n + 256 * ARGMAX_U - 1) / (256 * ARGMAX_U);
-    if (g < 1) g = 1;
-    if (g > ARGMAX_PARTS) g = ARGMAX_PARTS;
-    hipLaunchKernelGGL(k_argmax, dim3(g), dim3(256), 0, s, x, n, (uint32_t *)scratch, out);
-    return hipGetLastError();
+    auto go = [&](auto kern, uint32_t per) -> hipError_t {   // one round of `per` elements per workgroup, if it can
+        uint32_t g = (n + per - 1) / per;
+        if (g < 1) g = 1;
+        if (g > ARGMAX_PARTS) g = ARGMAX_PARTS;
+        hipLaunchKernelGGL(kern, dim3(g), dim3(256), 0, s, x, n, (uint32_t *)scratch, out);
+        return hipGetLastError();
+    };
+    // Half as many workgroups of eight loads a thread where they are many: each
+    // costs the count word an atomic and the last one a partial (65536: 3.76 us,
+    // with four loads 3.89; 151936: 4.14 and 4.84; 256000: 4.73 and 6.03).
+    return n < 65536 ? go(k_argmax<4>, 1024) : go(k_argmax<8>, 2048);
 }
 
 }  // namespace kq

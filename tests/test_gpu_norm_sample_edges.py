@@ -35,7 +35,8 @@ def test_norm_edges(hip, oracle, n):
     assert np.array_equal(out.download(np.uint32, n), oracle.rmsnorm(sx, sx, 1e-6).view(np.uint32))
 
 
-@pytest.mark.parametrize("n", [1, 63, 256, 257, 1023, 1024, 1025, 4096, 4097, 262144, 262145, 600001])
+@pytest.mark.parametrize("n", [1, 63, 256, 257, 1023, 1024, 1025, 4096, 4097, 65535, 65536, 67583, 262144, 262145,
+                               524288, 524289, 600001])
 def test_argmax_edges(hip, n):
     print(f"[argmax_edges] n={n}", flush=True)
     rng = np.random.default_rng(n)
