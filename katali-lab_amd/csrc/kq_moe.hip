@@ -3184,9 +3184,13 @@ static hipError_t go_b_run(const MoeArgs &a, uint32_t n_slots, const BPlan &pl, 
     // slots, have their own kernel (two slots of 14336, Q6_K: 25.8 -> 22.2 us;
     // six of 9728, Q4_K: 39.8 -> 18.0; ten of 4096, Q4_K: 38.1 -> 14.2). One
     // slot (a dense FFN) has one pair per wave there and gains nothing: 10.9
-    // us here at 12288, 11.4 there. Both give a pair the same lane split, the
-    // grouped kernels' too, so its sum has the same bits in all of them.
-    if (pl.key == 0 || (pl.key >= 16 * 8 && n_slots > 1)) return launch_moe_down_wide(a, n_slots, s);
+    // us here at 12288, 11.4 there; nor have fewer than four rows per CU, each
+    // with every slot's h to stage (layers of two slots of 14336: hidden 512
+    // 17.0 us here, 19.4 there; 1024 21.5 and 21.7, of four slots 40.4 and
+    // 34.7). Both give a pair the same lane split, the grouped kernels' too, so
+    // its sum has the same bits in all of them.
+    const bool wide = n_slots > 1 && a.hidden >= 4u * (uint32_t)device_cu_count();
+    if (pl.key == 0 || (pl.key >= 16 * 8 && wide)) return launch_moe_down_wide(a, n_slots, s);
     return a.down_type == T_Q6_K ? go_b_any<Q6K>(a, n_slots, pl, s) : go_b_any<Q4K>(a, n_slots, pl, s);
 }
 

@@ -32,6 +32,8 @@ CASES = [
     (256, 14336, 8, 8, False, Q4_K),     # h near the LDS limit
     (4096, 4352, 2, 2, False, Q6_K),     # 8 rows per workgroup
     (4096, 4608, 2, 2, True, Q4_K),
+    (1024, 4352, 4, 2, False, Q6_K),     # the fewest rows that take it at two slots, padded
+    (1024, 13824, 2, 2, False, Q6_K),
 ]
 
 
