@@ -58,13 +58,17 @@ __device__ __forceinline__ void dw_put_h(uint8_t *lds, uint32_t first, uint32_t 
     if ((r & 1) == 0) *x.d8(grp) = h2f(h.d);   // both halves of a block share it
 }
 
-template <class QD, int N>
+// PACK: the slots' h without gaps (DownPlan). Otherwise a slot starts with a
+// tile, and an item's place in it is one for all pairs: formed per pair it cost
+// layers of two Q4_K slots 0.1 to 0.2 us of 15 to 17.
+template <class QD, int N, bool PACK>
 __global__ void __launch_bounds__(DW_MAX_NT) k_moe_down_wide(MoeArgs a, uint32_t rpw, uint32_t inv_rpw, uint32_t n_slots,
                                                               uint32_t log2s) {
     extern __shared__ __align__(16) uint8_t lds[];
     using X = XLds<QD, 1>;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = blockDim.x;
     const uint32_t nb = a.ffn / 256, items = nb * QD::IPB;
+    const uint32_t slot_bytes = PACK ? 0 : X::bytes(items), slot_items = PACK ? items : 0;
     // the normed layer's exchange generation, read now and advanced at the
     // end, as kernel B does
     uint32_t gen = ld_dev(a.router ? a.fsync + 1 : (uint32_t *)a.route_ids);
@@ -100,12 +104,13 @@ __global__ void __launch_bounds__(DW_MAX_NT) k_moe_down_wide(MoeArgs a, uint32_t
     __builtin_amdgcn_sched_barrier(0);   // every weight load is out before h is staged
 #pragma unroll
     for (int i = 0; i < DW_HT; i++)
-        if (const uint32_t t = tid + nt * i; t < ntask) dw_put_h<QD>(lds, t / per * items, t % per, hv[i]);
+        if (const uint32_t t = tid + nt * i; t < ntask)
+            dw_put_h<QD>(lds + t / per * slot_bytes, t / per * slot_items, t % per, hv[i]);
     for (uint32_t t = tid + nt * DW_HT; t < ntask; t += nt)
-        dw_put_h<QD>(lds, t / per * items, t % per, dw_load_h(a.hq8, t));
+        dw_put_h<QD>(lds + t / per * slot_bytes, t / per * slot_items, t % per, dw_load_h(a.hq8, t));
     __syncthreads();
 
-    float *res = (float *)(lds + X::bytes(n_slots * items));   // [row][slot]
+    float *res = (float *)(lds + (PACK ? X::bytes(n_slots * items) : n_slots * slot_bytes));   // [row][slot]
     float acc = 0.0f;
     // batches of a pair, then the next pair, in one loop with one load: two
     // loads (or a nested loop) cost a second set of raw registers
@@ -114,7 +119,7 @@ __global__ void __launch_bounds__(DW_MAX_NT) k_moe_down_wide(MoeArgs a, uint32_t
 #pragma unroll
         for (int i = 0; i < N; i++) {
             const uint32_t at = s + S * (i0 + i), item = min(at, items - 1);
-            const X x(lds, sl * items + item);
+            const X x(lds + sl * slot_bytes, sl * slot_items + item);
             const float v = item_dot<1>(QD::full(raw[i]), (int)(item % QD::IPB), x);
             acc += at < items ? v : 0.0f;
             asm volatile("" : "+v"(acc)::"memory");   // one item's h in registers at a time
@@ -160,7 +165,8 @@ static hipError_t down_wide(const MoeArgs &a, uint32_t n_slots, hipStream_t st) 
     if (!down_plan(QD::TYPE == T_Q6_K, a.hidden, a.ffn, n_slots, (uint32_t)device_cu_count(), p))
         return hipErrorInvalidValue;
     return with_n<dw_nmax<QD>()>(p.N, [&](auto n) -> hipError_t {
-        auto kern = k_moe_down_wide<QD, decltype(n)::value>;
+        constexpr int N = decltype(n)::value;
+        auto kern = p.pack ? k_moe_down_wide<QD, N, true> : k_moe_down_wide<QD, N, false>;
         const hipError_t e = lds_limit(kern, p.lds);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(kern, dim3((a.hidden + p.rpw - 1) / p.rpw), dim3(64 * p.nw), p.lds, st, a, p.rpw, p.inv_rpw,

@@ -37,7 +37,7 @@ DOWN_DRIVER = r"""
 #include "kq_plan.h"
 // every shape of rows above four blocks that the layer's LDS rule admits
 int main() {
-    unsigned long n = 0, ragged = 0, bad = 0;
+    unsigned long n = 0, ragged = 0, packed = 0, bad = 0;
     for (unsigned cus : {20u, 32u, 38u, 64u, 80u, 228u, 256u, 304u})
         for (unsigned hidden : {256u, 512u, 1024u, 2048u, 4096u})
             for (unsigned nb = 5; nb <= 64; nb++)
@@ -48,14 +48,17 @@ int main() {
                         bool ok = kq::down_plan(q6, hidden, ffn, slots, cus, p);
                         n++;
                         if (!ok) { bad++; continue; }
-                        const unsigned h = (slots * nb * ipb + 15) / 16 * 16 / ipb * 352;
+                        const unsigned tile = 16 / ipb * 352, gaps = slots * ((nb * ipb + 15) / 16) * tile;
+                        const unsigned h = p.pack ? (slots * nb * ipb + 15) / 16 * tile : gaps;
+                        packed += p.pack;
+                        if (p.pack && gaps + 4 * (slots + 17) < 100000) bad++;   // packed only near the limit
                         ok = p.lds <= 163840 && p.lds >= h + (p.rpw * slots + 17) * 4 && p.rpw >= 1 && p.rpw <= 64 * p.nw &&
                              p.nw >= 4 && p.nw <= 16 && p.S == (nb > 16 ? 64 : 4 * ipb) && p.N >= 1 && p.N <= (q6 ? 4 : 8);
                         for (unsigned pc = 0; pc < p.rpw * slots; pc++) ok = ok && pc * p.inv_rpw >> 20 == pc / p.rpw;
                         ragged += hidden % p.rpw != 0;
                         if (!ok) bad++;
                     }
-    printf("%lu %lu %lu\n", n, ragged, bad);
+    printf("%lu %lu %lu %lu\n", n, ragged, packed, bad);
     return 0;
 }
 """
@@ -84,8 +87,8 @@ def run_driver(tmp_path, code):
 
 
 def test_down_plan(tmp_path):
-    n, ragged, bad = map(int, run_driver(tmp_path, DOWN_DRIVER))
-    assert n > 10000 and ragged > 0 and bad == 0
+    n, ragged, packed, bad = map(int, run_driver(tmp_path, DOWN_DRIVER))
+    assert n > 10000 and ragged > 0 and 0 < packed < n // 10 and bad == 0
 
 
 def test_coresident_rule(tmp_path):
