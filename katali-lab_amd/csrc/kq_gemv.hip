@@ -13,9 +13,10 @@
 // by its converts and FMAs, about 110 per 18 bytes: 40000 x 5120 4.0 TB/s), by
 // launch, first loads and tail below about 20 MB. Row lengths that are no
 // power of two used to run a loop over items with one load in flight and as
-// few as 4 lanes per row (weights from memory: Q6_K 5120 x 13824, fp32, 50.4 us,
-// now 20.0; q, k, v of 2560 columns 10.1, now 5.9; weights in the cache: the
-// first 37.2, now 16.8, and Q4_K 9731 x 2560, q8_1, 7.1, now 5.2).
+// few as 4 lanes per row (weights from memory: Q6_K 5120 x 13824, fp32, 50.3 us,
+// now 20.1; Q4_K 9731 x 2560, quantizing, 8.9, now 5.6; q, k, v of 2560 columns
+// 10.1, now 5.9; weights in the cache, the first two 37.2, now 16.6, and 7.1,
+// now 5.2).
 #include "kq_device.h"
 #include "kq_items.h"
 #include "kq_launch.h"
